@@ -28,6 +28,36 @@ ApplyLauncher launcher_for(int N)
   }
   return nullptr;
 }
+
+ApplyLauncher chain_launcher_for(int N)
+{
+  switch (N)
+  {
+  case 2: return launch_chain_n2;
+  case 3: return launch_chain_n3;
+  case 4: return launch_chain_n4;
+  case 5: return launch_chain_n5;
+  case 6: return launch_chain_n6;
+  case 7: return launch_chain_n7;
+  case 8: return launch_chain_n8;
+  case 9: return launch_chain_n9;
+  }
+  return nullptr;
+}
+
+// The launcher of a validated request: a gathered apply through the atomic
+// scatter goes to the chain kernel where that is the faster one.
+ApplyLauncher pick_launcher(const ApplyReq& r)
+{
+  if (r.N > FEMTC_MAX_FUSED_DEGREE + 1)
+    return r.N <= FEMTC_MAX_DEGREE + 1 ? launch_apply_general : nullptr;
+  const bool atomic = r.gather && !r.reference_mode && !r.blocked &&
+                      !r.assembled && !r.structured_direct && !r.zrun &&
+                      !r.eo_tab && !r.energy;
+  if (atomic && chain_pays(r.op, r.dtype == FEMTC_F64, r.N, r.Q))
+    return chain_launcher_for(r.N);
+  return launcher_for(r.N);
+}
 } // namespace
 
 int fail(int status, const std::string& msg)
@@ -82,9 +112,7 @@ int run(const ApplyReq& r)
     return fail(FEMTC_ERR_INVALID_ARGUMENT,
                 "G must be aligned to two elements (16 bytes for FP64, 8 for "
                 "FP32)");
-  ApplyLauncher f = launcher_for(r.N);
-  if (!f && r.N <= FEMTC_MAX_DEGREE + 1)
-    f = launch_apply_general; // degrees above the fused kernels
+  ApplyLauncher f = pick_launcher(r);
   if (!f)
     return fail(FEMTC_ERR_DEGREE_NOT_SUPPORTED, "degree not supported");
   const int st = f(r);

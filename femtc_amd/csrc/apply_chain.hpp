@@ -1,0 +1,393 @@
+// Chain kernel: the continuous operator through any dofmap, with the faces
+// that consecutive cells share summed in LDS.
+//
+// What bounds the gathered kernel of apply_kernel.hpp is mostly its scatter:
+// N^3 memory-side atomics per cell in runs of N addresses (61-77 G/s; runs of
+// 33 sustain 141 G/s).  Mesh numberings, lexicographic or in the order a
+// reader meets the cells, mostly list neighbours one after another, so here
+// one workgroup takes a chain of S consecutive cells.  Each cell's right
+// face (c = P) and the next cell's left face (c = 0) share one slot of a box
+// [N][N][S P + 1] in LDS wherever the dofmap gives both the same dofs; the
+// box then goes to y with one atomic per slot, consecutive lanes on
+// consecutive dofs.
+//
+//  * Any dofmap is correct: a left-face dof that is not its left neighbour's
+//    right-face dof is added to y on its own.  The check reads only the
+//    dofmap entries that the neighbour's lanes read anyway.
+//  * No LDS atomics: slot c >= 1 of a cell belongs to that cell (its lanes
+//    store it), and after a barrier the left faces are added to their
+//    neighbours' slots, one owner each.  LDS FP32 atomics made the P=6 FP32
+//    K+M pass 385 us against 248.
+//  * The write order of the box follows the numbering: along z through the
+//    whole chain when the middle row continues from cell to cell, else cell
+//    by cell (a reader's numbering gives each cell's new dofs one run).
+//
+// Cell groups.  Up to Q = 8 every wave takes 64 / Q^2 cells of the chain in
+// its own LDS work area with wave-local stage syncs.  At Q = 6 that leaves 28
+// of 64 lanes idle, so the workgroup's 4 waves take 7 cells together (252 of
+// 256 lanes): affine FP64 K+M at P=5, 97,290 cells, 248 -> 218 us.  At Q = 5
+// and 7 (50 and 49 lanes) the same packing was neutral or slower.
+//
+// Measured (MI355X, overwriting applies with the clear of y, us, the
+// gathered kernel of apply_kernel.hpp against this one): FP32 mass P=3 Q=5,
+// 61x67x71 cells, lexicographic 288 -> 118 and reader order 361 -> 120; FP32
+// stiffness P=4, 64^3, 485 -> 242; affine FP64 K+M P=5, 45x46x47, 288 -> 236;
+// FP64 mass P=7, 40x41x42, 417 -> 301.
+#pragma once
+
+#include "cell_chain.hpp"
+
+namespace femtc
+{
+
+// Waves of a chain workgroup: 4, as far as their work areas and the box leave
+// a second workgroup room on the CU; 2 where a wave holds 7 or 16 cells and
+// two already make long rows (affine FP64 stiffness P=2, 1.6e7 dofs: 403 ->
+// 371 us; mass P=1: 627 -> 557).
+template <typename T, int Q, int OP>
+constexpr int chain_waves()
+{
+  if (Q <= 3)
+    return 2;
+  return sizeof(T) == 8 && Q == 8 && OP != OP_MASS && OP != OP_MASS_AFF ? 3 : 4;
+}
+
+template <typename T, int N, int Q, int OP>
+struct ChainShape
+{
+  using Ch = CellChain<T, N, Q, OP, false>;
+  static constexpr int P = N - 1;
+  static constexpr int BT = 64 * chain_waves<T, Q, OP>();
+  static constexpr bool PACK = Q == 6;         // cells straddle waves
+  static constexpr int GT = PACK ? BT : 64;    // threads of a cell group
+  static constexpr int NG = BT / GT;           // groups
+  static constexpr int CPB = GT / (Q * Q);     // cells of a group
+  static constexpr int S = NG * CPB;           // cells of the chain
+  static constexpr int Z = S * P + 1;          // dofs of a box row
+  // row (a, b) at a SA + b Z: SA spreads the lanes (a, c) of a store over
+  // the LDS banks
+  static constexpr int SLOTS = sizeof(T) == 8 ? 32 : 64;
+  static constexpr int SA = N * Z + ((N - N * Z) % SLOTS + SLOTS) % SLOTS;
+  static constexpr int BOX = N * SA;
+  static constexpr int WC = Ch::template wcell<CPB>();
+  // geometry of a group in pieces of two elements, in two halves of
+  // qa-planes [0, QA1) and [QA1, Q)
+  static constexpr int QA1 = geometry_split<Q>();
+  static constexpr int GP0 = Ch::GEO ? 3 * QA1 * Q * Q * CPB : 0;
+  static constexpr int GP1 = Ch::GEO ? 3 * (Q - QA1) * Q * Q * CPB : 0;
+  static constexpr int GPT0 = (GP0 + GT - 1) / GT, GPT1 = (GP1 + GT - 1) / GT;
+  static constexpr int WORK = CPB * WC > 2 * GP0 ? CPB * WC : 2 * GP0;
+  static constexpr int LDSW = (WORK + 1) / 2; // pieces per group
+  static constexpr size_t LDS = sizeof(Piece<T>) * (size_t)NG * LDSW +
+                                (sizeof(T) + sizeof(int32_t)) * (size_t)BOX;
+};
+
+template <typename T, int N, int Q, int OP>
+__global__ void __launch_bounds__((64 * chain_waves<T, Q, OP>()))
+    chain_cells(const T* __restrict__ tab, const T* __restrict__ x,
+                T* __restrict__ y, const T* __restrict__ G,
+                const T* __restrict__ detJw, const int32_t* __restrict__ dofmap,
+                long long num_cells, int nblk, const int* __restrict__ skip)
+{
+  if (skip && *skip)
+    return;
+  using Sh = ChainShape<T, N, Q, OP>;
+  using Ch = typename Sh::Ch;
+  constexpr int P = N - 1, NN = N * N, N3 = N * NN, Q2 = Q * Q, Q3 = Q2 * Q;
+  constexpr int GT = Sh::GT, CPB = Sh::CPB, Z = Sh::Z, SA = Sh::SA;
+  extern __shared__ __align__(16) unsigned char femtc_lds_dyn[];
+  // contiguous ranges of chains per XCD (workgroups are dealt round-robin):
+  // neighbouring chains share x lines and y lines in one L2
+  const long long per = (nblk + 7) / 8;
+  const long long blk = (long long)(blockIdx.x % 8) * per + blockIdx.x / 8;
+  if (blk >= nblk)
+    return; // uniform over the workgroup
+  const int grp =
+      Sh::PACK ? 0 : __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  Piece<T>* Ls = reinterpret_cast<Piece<T>*>(femtc_lds_dyn) + grp * Sh::LDSW;
+  T* box = reinterpret_cast<T*>(reinterpret_cast<Piece<T>*>(femtc_lds_dyn) +
+                                Sh::NG * Sh::LDSW);
+  int32_t* gid = reinterpret_cast<int32_t*>(box + Sh::BOX);
+  auto sync = [] {
+    if constexpr (Sh::PACK)
+      lds_barrier();
+    else
+      stage_sync<true>();
+  };
+
+  // the chain's cells, this group's first one, and this lane's; a lane
+  // without a cell repeats the chain's last one and stores nothing
+  const long long chain0 = blk * Sh::S;
+  const int ncell =
+      num_cells - chain0 < Sh::S ? (int)(num_cells - chain0) : Sh::S;
+  const int k0 = grp * CPB;
+  const int tid = (int)(threadIdx.x & (GT - 1));
+  const int lc = tid / Q2, ln = tid - lc * Q2;
+  const bool live = lc < CPB && k0 + lc < ncell;
+  const int k = live ? k0 + lc : ncell - 1;
+  const long long cell = chain0 + k;
+  T* Xc = reinterpret_cast<T*>(Ls) + (lc < CPB ? lc : 0) * Sh::WC;
+  // thread roles (lanes past a role's lines take its line 0)
+  const int ln1 = ln < NN ? ln : 0, ln2 = ln < N * Q ? ln : 0;
+  const int r1a = ln1 / N, r1c = ln1 - r1a * N; // F1/B1: (a, c)
+  const int r2q = ln2 / N, r2a = ln2 - r2q * N; // F2/B2: (qb, a)
+  const int q3b = ln / Q, q3c = ln - q3b * Q;   // F3/B3: (qb, qc)
+  const int yo3 = q3b * Ch::YQ + q3c;
+  const bool on1 = live && ln < NN, on2 = live && ln < N * Q;
+  const int slot0 = r1a * SA + k * P + r1c;
+
+  // ---------------- loads ----------------------------------------------
+  typename Ch::Tab tabs;
+  tabs.load(tab);
+  const int32_t* dm = dofmap + cell * N3 + r1a * NN;
+  int32_t idx[N];
+#pragma unroll
+  for (int b = 0; b < N; ++b)
+    idx[b] = dm[r1c + b * N];
+  // bit b: (a, b, 0) is not the left neighbour's (a, b, P)
+  const bool face = r1c == 0 && k > 0;
+  unsigned miss = 0;
+  {
+    const int off = face ? P - N3 : r1c;
+#pragma unroll
+    for (int b = 0; b < N; ++b)
+      miss |= (dm[off + b * N] != idx[b] ? 1u : 0u) << b;
+  }
+  T u[N];
+#pragma unroll
+  for (int b = 0; b < N; ++b)
+    u[b] = x[idx[b]];
+  Piece<T> gp0[Ch::GEO ? Sh::GPT0 : 1], gp1[Ch::GEO ? Sh::GPT1 : 1];
+  if constexpr (Ch::GEO)
+  {
+    // lane-contiguous pieces of the group's cells, as they are laid out in
+    // LDS: [cell][plane][qb][qc][6]
+    const int left = ncell - 1 - k0; // last cell, from the group's first
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+    {
+      const int pc = 3 * (h ? Q - Sh::QA1 : Sh::QA1) * Q2; // pieces per cell
+      const int tot = h ? Sh::GP1 : Sh::GP0;
+      const T* Gh = G + (chain0 + k0) * 6 * Q3 + (h ? 6 * Sh::QA1 * Q2 : 0);
+#pragma unroll
+      for (int i = 0; i < (h ? Sh::GPT1 : Sh::GPT0); ++i)
+      {
+        int p = i * GT + tid;
+        if (GT * (i + 1) > tot)
+          p = p < tot ? p : tot - 1;
+        const int c = CPB > 1 ? (int)((unsigned)p / (unsigned)pc) : 0;
+        const int r = p - c * pc;
+        const Piece<T>* src = reinterpret_cast<const Piece<T>*>(
+            Gh + (long long)(c < left ? c : left) * 6 * Q3);
+        (h ? gp1[i] : gp0[i]) = stream_load(src + r);
+      }
+    }
+  }
+  T cg[Ch::AFF ? CELLGEO : 1];
+  T wbc = T(1);
+  if constexpr (Ch::AFF)
+  {
+#pragma unroll
+    for (int i = 0; i < CELLGEO; ++i)
+      cg[i] = G[cell * CELLGEO + i];
+    wbc = tab[Ch::WOFF + q3b] * tab[Ch::WOFF + q3c];
+  }
+  T dw[Ch::MASSTERM ? Q : 1];
+  if constexpr (Ch::MASSTERM && !Ch::AFF)
+  {
+    const T* Dp = detJw + cell * Q3 + ln;
+#pragma unroll
+    for (int q = 0; q < Q; ++q)
+      dw[q] = stream_load(Dp + q * Q2);
+  }
+  if (on1)
+  {
+#pragma unroll
+    for (int b = 0; b < N; ++b)
+      if (!((miss >> b) & 1u))
+        gid[slot0 + b * Z] = idx[b];
+  }
+
+  // ---------------- the cells' contraction chain ------------------------
+  Ch::f1(tabs, u, Xc, r1a, r1c, on1);
+  sync();
+  T bpp[Q], bpg[Q], bgp[Q];
+  Ch::f2(tabs, Xc, r2q, r2a, bpp, bpg, bgp);
+  sync(); // X is read; Y overwrites the same LDS
+  Ch::f2_store(Xc, r2q, r2a, on2, bpp, bpg, bgp);
+  sync();
+  T ipp[N], ipg[N], igp[N];
+  Ch::f3_load(Xc, yo3, ipp, ipg, igp);
+  sync();
+  if constexpr (Ch::GEO)
+  {
+#pragma unroll
+    for (int i = 0; i < Sh::GPT0; ++i)
+      if (i * GT + tid < Sh::GP0)
+        Ls[i * GT + tid] = gp0[i];
+    sync();
+  }
+  T uq[Q], da[Q], db[Q], dc[Q];
+  Ch::f3(tabs, ipp, ipg, igp, uq, da, db, dc);
+  T va[Q], vb[Q], vc[Q], vm[Q];
+  auto point = [&](int q, int qa0, int planes) {
+    T g[6];
+    T dwq = T(0), w = T(0);
+    if constexpr (Ch::GEO)
+    {
+      const Piece<T>* Lg = Ls + (lc < CPB ? lc : 0) * 3 * planes * Q2 +
+                           ((q - qa0) * Q2 + ln) * 3;
+#pragma unroll
+      for (int j = 0; j < 3; ++j)
+      {
+        const Piece<T> pc = Lg[j];
+        g[2 * j] = pc.x;
+        g[2 * j + 1] = pc.y;
+      }
+    }
+    if constexpr (Ch::AFF)
+      w = tab[Ch::WOFF + q] * wbc;
+    else if constexpr (Ch::MASSTERM)
+      dwq = dw[q];
+    Ch::point(q, g, dwq, cg, w, uq, da, db, dc, va, vb, vc, vm);
+  };
+#pragma unroll
+  for (int q = 0; q < Sh::QA1; ++q)
+    point(q, 0, Sh::QA1);
+  if constexpr (Ch::GEO)
+  {
+    sync();
+#pragma unroll
+    for (int i = 0; i < Sh::GPT1; ++i)
+      if (i * GT + tid < Sh::GP1)
+        Ls[i * GT + tid] = gp1[i];
+    sync();
+  }
+#pragma unroll
+  for (int q = Sh::QA1; q < Q; ++q)
+    point(q, Sh::QA1, Q - Sh::QA1);
+  T ra_[N], rb_[N], rc_[N];
+  Ch::b3(tabs, va, vb, vc, vm, ra_, rb_, rc_);
+  if constexpr (Ch::GEO)
+    sync(); // the geometry in LDS is consumed; Y may be rewritten
+  Ch::b3_store(Xc, yo3, live, ra_, rb_, rc_);
+  sync();
+  T ra[Q], rb[Q], rc[Q];
+  Ch::b2_load(Xc, r2q, r2a, ra, rb, rc);
+  sync(); // Y is read; X overwrites the same LDS
+  Ch::b2(tabs, ra, rb, rc, Xc, r2q, r2a, on2);
+  sync();
+  T w[N];
+  Ch::b1(tabs, Xc, r1a, r1c, w);
+
+  // ---------------- the chain's box, then y ------------------------------
+  if (on1 && !face)
+  {
+#pragma unroll
+    for (int b = 0; b < N; ++b)
+      box[slot0 + b * Z] = w[b];
+  }
+  lds_barrier();
+  if (on1 && face)
+  {
+#pragma unroll
+    for (int b = 0; b < N; ++b)
+    {
+      if ((miss >> b) & 1u)
+        atomic_add(y + dm[b * N], w[b]);
+      else
+        box[slot0 + b * Z] += w[b];
+    }
+  }
+  lds_barrier();
+  const int zlen = ncell * P + 1;
+  const int mid = SA + Z; // row (1, 1)
+  const bool along_z = ncell < 2 || gid[mid + P + 1] == gid[mid + P] + 1;
+  for (int i = threadIdx.x; i < NN * Z; i += Sh::BT)
+  {
+    int ab, z;
+    if (along_z)
+    {
+      ab = i / Z;
+      z = i - ab * Z;
+    }
+    else if (i < NN)
+    {
+      ab = i; // the first cell's left face
+      z = 0;
+    }
+    else
+    {
+      const int j = i - NN;
+      const int kc = j / (NN * P), r = j - kc * (NN * P);
+      ab = r / P;
+      z = kc * P + 1 + (r - ab * P);
+    }
+    const int a = ab / N;
+    const int s = a * SA + (ab - a * N) * Z + z;
+    if (z < zlen)
+      atomic_add(y + gid[s], box[s]);
+  }
+}
+
+template <typename T, int N, int Q, int OP>
+int launch_chain(const ApplyReq& r)
+{
+  if constexpr (!chain_pays(OP, sizeof(T) == 8, N, Q))
+    return FEMTC_ERR_INVALID_ARGUMENT;
+  else
+  {
+    using Sh = ChainShape<T, N, Q, OP>;
+    if (!r.gather || r.reference_mode || r.energy)
+      return FEMTC_ERR_INVALID_ARGUMENT;
+    const long long nblk = (r.num_cells + Sh::S - 1) / Sh::S;
+    if (nblk == 0)
+      return FEMTC_OK;
+    if (nblk > 0x7ffffff0LL)
+      return FEMTC_ERR_INVALID_ARGUMENT;
+    static_assert(Sh::LDS <= 64 * 1024, "chain workgroup LDS");
+    hipLaunchKernelGGL((chain_cells<T, N, Q, OP>),
+                       dim3((unsigned)(8 * ((nblk + 7) / 8))), dim3(Sh::BT),
+                       Sh::LDS, r.stream, (const T*)r.tab, (const T*)r.x,
+                       (T*)r.y, (const T*)r.G, (const T*)r.detJw, r.dofmap,
+                       (long long)r.num_cells, (int)nblk, r.skip);
+    return hip_status(hipGetLastError());
+  }
+}
+
+template <typename T, int N, int Q>
+int chain_op(const ApplyReq& r)
+{
+  switch (r.op)
+  {
+  case OP_MASS: return launch_chain<T, N, Q, OP_MASS>(r);
+  case OP_STIFF: return launch_chain<T, N, Q, OP_STIFF>(r);
+  case OP_KPM: return launch_chain<T, N, Q, OP_KPM>(r);
+  case OP_MASS_AFF: return launch_chain<T, N, Q, OP_MASS_AFF>(r);
+  case OP_STIFF_AFF: return launch_chain<T, N, Q, OP_STIFF_AFF>(r);
+  case OP_KPM_AFF: return launch_chain<T, N, Q, OP_KPM_AFF>(r);
+  }
+  return FEMTC_ERR_INVALID_ARGUMENT;
+}
+
+template <int N, int Q>
+int chain_dtype(const ApplyReq& r)
+{
+  return r.dtype == FEMTC_F64 ? chain_op<double, N, Q>(r)
+                              : chain_op<float, N, Q>(r);
+}
+
+// Q in {N, N+1, N+2}
+template <int N>
+int chain_q(const ApplyReq& r)
+{
+  switch (r.Q - N)
+  {
+  case 0: return chain_dtype<N, N>(r);
+  case 1: return chain_dtype<N, N + 1>(r);
+  case 2: return chain_dtype<N, N + 2>(r);
+  }
+  return FEMTC_ERR_INVALID_ARGUMENT;
+}
+
+} // namespace femtc

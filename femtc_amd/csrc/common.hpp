@@ -95,6 +95,35 @@ constexpr int SCATTER_STRUCT = -2;
 // BW template value of the structured z-run scatter (ApplyReq::zrun).
 constexpr int SCATTER_ZRUN = -3;
 
+// Where the chain kernel (apply_chain.hpp) runs a gathered apply instead of
+// the atomic scatter of apply_kernel.hpp: where the N^3 atomics per cell, not
+// the contractions or the geometry stream, set the time.  Measured over
+// every degree, Q and operator on meshes of 3e6 and 1.6e7 dofs (MI355X, time
+// of the atomic scatter over the chain's, both with the clear of y):
+//   mass                           1.2-4.0 at every Q <= 8
+//   affine FP32                    1.1-3.5 at every Q <= 8
+//   affine FP64 stiffness, K+M     1.2-2.7 at Q = N <= 7 (0.97-1.05 at N = 8),
+//                                  1.0-1.7 at Q = N + 1 with N = 3..6
+//                                  (elsewhere 0.90-1.11), 0.9-1.3 at Q = N + 2
+//   FP32 stiffness, K+M            1.1-2.4, but 0.94-1.03 at Q = N + 2 with
+//                                  N = 2, 3, 5
+//   FP64 stiffness, K+M            1.05-2.3 at Q = N <= 5 (K+M at P=2: 0.94
+//                                  lexicographic, 1.7 in reader order),
+//                                  0.91-1.06 elsewhere
+// A cell of Q >= 9 does not fit one wave: the chain would be too short.
+constexpr bool chain_pays(int op, bool f64, int N, int Q)
+{
+  if (Q > 8)
+    return false;
+  if (op == OP_MASS || op == OP_MASS_AFF)
+    return true;
+  const bool affine = op == OP_STIFF_AFF || op == OP_KPM_AFF;
+  if (!f64)
+    return affine || Q < N + 2 || N == 4 || N > 5;
+  return affine ? (Q == N && N < 8) || (Q == N + 1 && N > 2 && N < 7)
+                : Q == N && N <= 5 && !(op == OP_KPM && N == 3);
+}
+
 // Cells per workgroup of the fused cell kernel (Q^2 threads per cell):
 // one wave of whole cells up to Q = 8.  At Q = 9 one cell in a 2-wave
 // workgroup would leave 47 of its 128 lanes idle; three cells take 243 of
@@ -188,6 +217,17 @@ int launch_apply_n6(const ApplyReq&);
 int launch_apply_n7(const ApplyReq&);
 int launch_apply_n8(const ApplyReq&);
 int launch_apply_n9(const ApplyReq&);
+// Chain kernels (apply_chain.hpp), one translation unit per N: gathered
+// applies in correct mode without energies; FEMTC_ERR_INVALID_ARGUMENT where
+// the kernels of launch_apply_n<N> are the faster ones (chain_pays).
+int launch_chain_n2(const ApplyReq&);
+int launch_chain_n3(const ApplyReq&);
+int launch_chain_n4(const ApplyReq&);
+int launch_chain_n5(const ApplyReq&);
+int launch_chain_n6(const ApplyReq&);
+int launch_chain_n7(const ApplyReq&);
+int launch_chain_n8(const ApplyReq&);
+int launch_chain_n9(const ApplyReq&);
 // N = 10..26 (apply_general.hip); also accepts smaller N
 int launch_apply_general(const ApplyReq&);
 // Line kernels, N = 10..26 (apply_line.hpp); max_lds = the device's LDS

@@ -369,8 +369,11 @@ int plan_request(const femtc_plan* pl, int op, int dtype, int nq,
   r.Q = nq;
   r.gather = 1;
   r.tab = tables;
-  // the even-odd instances cover the direct and assembled scatters
-  r.eo_tab = (s.x == 0 || s.x == -1) && nq == r.N ? eo : nullptr;
+  // the even-odd instances cover the direct and assembled scatters; where
+  // the chain kernel takes the direct one, its merged faces are worth more
+  // than half-size products
+  const bool direct_eo = s.x == 0 && !chain_pays(op, dtype == FEMTC_F64, r.N, nq);
+  r.eo_tab = (direct_eo || s.x == -1) && nq == r.N ? eo : nullptr;
   r.x = x;
   r.y = y;
   r.G = G;

@@ -1,0 +1,110 @@
+"""The chain kernel behind the one-shot gathered applies: every kind of
+numbering it must merge or must not merge faces for, chains that end short,
+cells straddling waves (Q = 6), overwrite and accumulate, against the oracle.
+
+The kernel sums the same products as the atomic scatter in another order, so
+the bars are those of the gathered applies: 1e-12 (FP64), 1e-5 (FP32)."""
+import numpy as np
+import pytest
+
+import femtc_amd as F
+import oracle as O
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+TOL = {torch.float64: 1e-12, torch.float32: 1e-5}
+
+
+def numbered(kind, dims, P, seed=1):
+    """(dofmap, number of dofs) of the box `dims`, in the numbering `kind`."""
+    nx, ny, nz = dims
+    nd = (P + 1) ** 3
+    dm = O.dofmap_structured(nx, ny, nz, P).reshape(-1, nd)
+    ng = (nx * P + 1) * (ny * P + 1) * (nz * P + 1)
+    rng = np.random.default_rng(seed)
+    if kind == "reader":  # dofs in the order the cells first meet them
+        _, first = np.unique(dm, return_index=True)
+        rank = np.empty(ng, dtype=np.int64)
+        rank[np.argsort(first)] = np.arange(ng)
+        dm = rank[dm]
+    elif kind == "relabelled":
+        dm = rng.permutation(ng)[dm]
+    elif kind == "shuffled":  # consecutive cells share a face by chance only
+        dm = dm[rng.permutation(len(dm))]
+    elif kind == "periodic":  # the last cell of a z-line closes on its first
+        last = dm.reshape(nx, ny, nz, P + 1, P + 1, P + 1)
+        last[:, :, -1, :, :, -1] = last[:, :, 0, :, :, 0]
+    elif kind == "partial":  # one edge of each face is not shared
+        for k in range(1, len(dm)):
+            cell = dm[k].reshape(P + 1, P + 1, P + 1)
+            cell[0, :, 0] = cell[0, ::-1, 0].copy()
+    return np.ascontiguousarray(dm.ravel(), dtype=np.int32), ng
+
+
+def check(op, P, Q, dims, kind, dtype, affine=False, accumulate=False):
+    N, C = P + 1, int(np.prod(dims))
+    dm, ng = numbered(kind, dims, P)
+    J = O.random_jacobians(5, C)
+    G, Dw = O.geometry_affine(J, Q)
+    tab = O.basis_tables(P, Q)
+    x = O.uniform(11, ng)
+    y0 = O.uniform(12, ng)
+    ref = O.global_operator(op, N, Q, tab, x, dm, G, Dw)
+    if accumulate:
+        ref = ref + y0
+
+    def dev(a):
+        return torch.from_numpy(np.ascontiguousarray(a)).to("cuda", dtype)
+
+    y = dev(y0)
+    code = {"mass": F.OP_MASS, "stiffness": F.OP_STIFFNESS,
+            "kpm": F.OP_KPM}[op]
+    ddm = torch.from_numpy(dm).cuda()
+    if affine:
+        cg = torch.empty(C * 7, device="cuda", dtype=dtype)
+        F.geometry_cell(torch.from_numpy(J).cuda(), cg)
+        F.global_apply_affine(code, dev(F.basis_tables_weights(P, Q)), dev(x),
+                              y, ddm, C, P, Q, cg, accumulate=accumulate)
+    else:
+        F.global_apply(code, dev(tab), dev(x), y, ddm, C, P, Q, G=dev(G),
+                       detJw=dev(Dw), accumulate=accumulate)
+    torch.cuda.synchronize()
+    got = y.double().cpu().numpy()
+    err = np.linalg.norm(got - ref) / np.linalg.norm(ref)
+    assert err <= TOL[dtype], (op, P, Q, dims, kind, dtype, err)
+
+
+KINDS = ["lex", "reader", "relabelled", "shuffled", "periodic", "partial"]
+# chains of 32, 14, 8, 7 (cells over the 4 waves at Q = 6), 4 and 3 cells:
+# lines shorter than, equal to and longer than a chain
+SHAPES = [(1, 2, (2, 2, 9)), (2, 3, (2, 3, 5)), (3, 5, (2, 2, 7)),
+          (4, 5, (1, 3, 8)), (5, 6, (2, 2, 5)), (3, 6, (1, 2, 4)),
+          (6, 7, (1, 2, 5)), (7, 8, (1, 2, 4))]
+
+
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("P,Q,dims", SHAPES)
+def test_numberings(P, Q, dims, kind):
+    for op in ("mass", "stiffness", "kpm"):
+        for dtype in (torch.float64, torch.float32):
+            check(op, P, Q, dims, kind, dtype)
+            check(op, P, Q, dims, kind, dtype, affine=True, accumulate=True)
+
+
+@pytest.mark.parametrize("P,Q", [(P, Q) for P in range(1, 9)
+                                 for Q in range(P + 1, min(P + 4, 10))])
+def test_chain_ends(P, Q):
+    """One cell, and counts around the chain's length."""
+    for nz in (1, 2, 3, 7, 8, 15, 33):
+        check("mass", P, Q, (1, 1, nz), "lex", torch.float64,
+              accumulate=nz % 2 == 1)
+        check("kpm", P, Q, (1, 1, nz), "reader", torch.float32, affine=True)
+
+
+def test_periodic_single_cell():
+    """A cell whose own right and left faces are the same dofs."""
+    for P, Q in ((1, 2), (4, 5), (5, 6), (7, 8)):
+        check("mass", P, Q, (2, 2, 1), "periodic", torch.float64)
+        check("stiffness", P, Q, (2, 2, 1), "periodic", torch.float32,
+              affine=True)
