@@ -36,15 +36,41 @@ namespace
 {
 
 constexpr int RB = 256;    // threads per block, vector kernels
-constexpr int NBLK = 1024; // blocks of the vector kernels (fixed: the partial
-                           // sums are always combined in the same order)
+// Most blocks of the vector kernels.  A solver's number (vec_blocks) depends
+// on its size alone, so its partial sums are always combined in the same
+// order.
+constexpr int NBLK = 1024;
 
+// Blocks of the vector kernels on n values: one value per thread while that
+// takes fewer than NBLK blocks.
+int vec_blocks(int64_t n)
+{
+  return (int)std::min<int64_t>(NBLK, std::max<int64_t>(1, (n + RB - 1) / RB));
+}
+
+// Operator energies that the update sums itself; more of them are combined
+// into block partials first (k_energy_partials).
+constexpr int64_t EPART_DIRECT = 4096;
+
+// The CG scalars.  An iteration is operator, update, p-update: every block of
+// the update computes alpha from the operator's energies, and every block of
+// the p-update computes beta and the convergence test from the update's
+// partials, each the same value in the same order; block 0 alone writes the
+// state.  No block reads a field that its own kernel writes (a block that did
+// could take another branch than its neighbours, or its own waves different
+// ones): the update reads done, rz_next and it and writes rz, it_pending,
+// alpha and epend; the p-update reads those and writes rz_next, it, rr,
+// status and done.
 struct PcgState
 {
-  double rz, rr, pAp, alpha, beta, tol2, rr0;
-  int it, maxit, done, status;
-  // alpha of this iteration is valid and e += alpha p is still to be
-  // applied (by k_pupdate, which reads p anyway)
+  double rz, rz_next, rr, pAp, alpha, tol2, rr0;
+  // iterations done (written by the p-update) and, as the p-update's blocks
+  // read it, before this one (copied by the update)
+  int it, it_pending;
+  int maxit, done, status;
+  // written by the update: 1 when alpha of this iteration is valid and e +=
+  // alpha p is still to be applied (by the p-update, which reads p anyway), 0
+  // when the solve was done before, -1 on a breakdown (p.Ap not positive)
   int epend;
 };
 
@@ -97,19 +123,40 @@ __device__ inline void store_partials(double (&v)[NV], double* part)
   }
 }
 
-// Combine the NBLK partials of NV sums (one block of RB threads).
-template <int NV>
-__device__ inline void combine_partials(const double* part, double (&v)[NV])
+// Combine the npart partials of NV sums (one block of BT threads); the result
+// is valid in thread 0.
+template <int NV, int BT = RB>
+__device__ inline void combine_partials(const double* part, int npart,
+                                        double (&v)[NV])
 {
 #pragma unroll
   for (int k = 0; k < NV; ++k)
   {
     double s = 0.0;
-    for (int j = threadIdx.x; j < NBLK; j += RB)
+    for (int j = threadIdx.x; j < npart; j += BT)
       s += part[k * NBLK + j];
     v[k] = s;
   }
-  block_sum<NV>(v);
+  block_sum<NV, BT>(v);
+}
+
+// The same with the result in every thread.
+template <int NV, int BT = RB>
+__device__ inline void combine_for_all(const double* part, int npart,
+                                       double (&v)[NV])
+{
+  __shared__ double all[NV];
+  combine_partials<NV, BT>(part, npart, v);
+  if (threadIdx.x == 0)
+  {
+#pragma unroll
+    for (int k = 0; k < NV; ++k)
+      all[k] = v[k];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < NV; ++k)
+    v[k] = all[k];
 }
 
 // The Jacobi preconditioner D^-1 of a PCG in precision V is held as
@@ -141,7 +188,7 @@ __device__ inline float precond_value(uint16_t d)
 
 #define GRID_LOOP(i, n)                                                      \
   for (int64_t i = (int64_t)blockIdx.x * RB + threadIdx.x; i < (n);          \
-       i += (int64_t)NBLK * RB)
+       i += (int64_t)gridDim.x * RB)
 
 // ---------------------------------------------------------------- PCG ----
 
@@ -169,15 +216,16 @@ __global__ void __launch_bounds__(RB)
 }
 
 __global__ void __launch_bounds__(RB)
-    k_reduce_start(const double* __restrict__ part, PcgState* st, double rtol,
-                   int maxit)
+    k_reduce_start(const double* __restrict__ part, int npart, PcgState* st,
+                   double rtol, int maxit)
 {
   double v[2];
-  combine_partials<2>(part, v);
+  combine_partials<2>(part, npart, v);
   if (threadIdx.x == 0)
   {
     PcgState s{};
     s.rz = v[0];
+    s.rz_next = v[0];
     s.rr = v[1];
     s.rr0 = v[1];
     s.tol2 = rtol * rtol * v[1];
@@ -196,8 +244,9 @@ __global__ void __launch_bounds__(RB)
   }
 }
 
-// First stage of p.Ap: the operator kernel's per-wave quadrature-point
-// energies p_e^T A_e p_e (npart of them) summed into NBLK block partials.
+// First stage of p.Ap for large problems: the operator kernel's per-wave
+// quadrature-point energies p_e^T A_e p_e (npart of them) summed into one
+// partial per block.
 __global__ void __launch_bounds__(RB)
     k_energy_partials(const double* __restrict__ e, int64_t npart,
                       double* __restrict__ part,
@@ -210,33 +259,33 @@ __global__ void __launch_bounds__(RB)
   store_partials<1>(s, part);
 }
 
-// alpha = r.z / p.Ap (block partials combined in a fixed order)
-__global__ void __launch_bounds__(RB)
-    k_alpha(const double* __restrict__ part, PcgState* st)
+// The update's first step: alpha = r.z / p.Ap from the energies (npart
+// values, combined in a fixed order by every block).  Returns false when
+// there is nothing to update: the solve is done, or breaks down here.
+template <int BT>
+__device__ inline bool update_alpha(const double* __restrict__ energy,
+                                    int npart, PcgState* st, double* alpha)
 {
   if (st->done)
   {
-    if (threadIdx.x == 0)
+    if (blockIdx.x == 0 && threadIdx.x == 0)
       st->epend = 0; // the last step's e += alpha p has been applied
-    return;
+    return false;
   }
+  const double rz = st->rz_next;
   double v[1];
-  combine_partials<1>(part, v);
-  if (threadIdx.x == 0)
+  combine_for_all<1, BT>(energy, npart, v);
+  const bool ok = v[0] > 0.0 && __builtin_isfinite(v[0]);
+  *alpha = rz / v[0];
+  if (blockIdx.x == 0 && threadIdx.x == 0)
   {
     st->pAp = v[0];
-    if (!(v[0] > 0.0) || !__builtin_isfinite(v[0]))
-    {
-      st->done = 1;
-      st->status = FEMTC_ERR_BREAKDOWN;
-      st->epend = 0;
-    }
-    else
-    {
-      st->alpha = st->rz / v[0];
-      st->epend = 1;
-    }
+    st->rz = rz;
+    st->it_pending = st->it;
+    st->alpha = *alpha;
+    st->epend = ok ? 1 : -1;
   }
+  return ok;
 }
 
 // r -= alpha Ap, Ap = 0 (ready for the next scatter); partials of r.z and
@@ -245,11 +294,13 @@ template <typename V>
 __global__ void __launch_bounds__(RB)
     k_update(V* __restrict__ r, V* __restrict__ Ap,
              const typename Precond<V>::T* __restrict__ dinv, int64_t n,
-             const PcgState* __restrict__ st, double* __restrict__ part)
+             const double* __restrict__ energy, int nenergy, PcgState* st,
+             double* __restrict__ part)
 {
-  if (st->done)
-    return;
-  const V a = (V)st->alpha;
+  double alpha;
+  if (!update_alpha<RB>(energy, nenergy, st, &alpha))
+    return; // uniform over the block
+  const V a = (V)alpha;
   double s[2] = {0.0, 0.0};
   GRID_LOOP(i, n)
   {
@@ -275,13 +326,13 @@ template <typename V, int P>
 __global__ void __launch_bounds__(ARB)
     k_assemble_update(const V* __restrict__ W, V* __restrict__ r,
                       const typename Precond<V>::T* __restrict__ dinv,
-                      LatticeGrid L,
-                      const PcgState* __restrict__ st,
-                      double* __restrict__ part)
+                      LatticeGrid L, const double* __restrict__ energy,
+                      int nenergy, PcgState* st, double* __restrict__ part)
 {
-  if (st->done)
-    return;
-  const V a = (V)st->alpha;
+  double alpha;
+  if (!update_alpha<ARB>(energy, nenergy, st, &alpha))
+    return; // uniform over the block
+  const V a = (V)alpha;
   double s[2] = {0.0, 0.0};
   const long long nrows = lattice_global_rows(L);
   const int NZ = L.ncz * P + 1;
@@ -290,7 +341,7 @@ __global__ void __launch_bounds__(ARB)
   // index arithmetic and the lattice row pointers live in scalar registers
   const int wave0 = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   for (long long row = (long long)blockIdx.x * (ARB / 64) + wave0;
-       row < nrows; row += (long long)NBLK * (ARB / 64))
+       row < nrows; row += (long long)gridDim.x * (ARB / 64))
   {
     const V* rows[4];
     const int mask = lattice_rows<V, P>(W, (int)row, L, rows);
@@ -314,55 +365,53 @@ __global__ void __launch_bounds__(ARB)
   store_partials<2, ARB>(s, part);
 }
 
-__global__ void __launch_bounds__(RB)
-    k_beta(const double* __restrict__ part, PcgState* st)
-{
-  if (st->done)
-    return;
-  double v[2];
-  combine_partials<2>(part, v);
-  if (threadIdx.x == 0)
-  {
-    const double rzn = v[0];
-    st->beta = rzn / st->rz;
-    st->rz = rzn;
-    st->rr = v[1];
-    st->it += 1;
-    if (!__builtin_isfinite(v[0]) || !__builtin_isfinite(v[1]))
-    {
-      st->done = 1;
-      st->status = FEMTC_ERR_BREAKDOWN;
-    }
-    else if (v[1] <= st->tol2)
-    {
-      st->done = 1;
-      st->status = FEMTC_OK;
-    }
-    else if (st->it >= st->maxit)
-    {
-      st->done = 1;
-      st->status = FEMTC_ERR_NOT_CONVERGED;
-    }
-  }
-}
-
-// e += alpha p (this iteration's step), then p = D^-1 r + beta p unless the
-// iteration ended the solve
+// beta and the convergence test from the update's npart partials (every
+// block the same), e += alpha p (this iteration's step), then p = D^-1 r +
+// beta p unless the iteration ended the solve.
 template <typename V>
 __global__ void __launch_bounds__(RB)
     k_pupdate(V* __restrict__ p, V* __restrict__ e, const V* __restrict__ r,
               const typename Precond<V>::T* __restrict__ dinv, int64_t n,
-              const PcgState* __restrict__ st)
+              const double* __restrict__ part, int npart, PcgState* st)
 {
-  if (!st->epend)
+  if (st->epend <= 0)
+  {
+    if (st->epend < 0 && blockIdx.x == 0 && threadIdx.x == 0)
+    {
+      st->status = FEMTC_ERR_BREAKDOWN;
+      st->done = 1;
+    }
     return;
+  }
+  const double rz = st->rz, tol2 = st->tol2;
   const V a = (V)st->alpha;
-  if (st->done)
+  double v[2];
+  combine_for_all<2>(part, npart, v);
+  const bool broken =
+      !__builtin_isfinite(v[0]) || !__builtin_isfinite(v[1]);
+  const bool met = v[1] <= tol2;
+  const int it = st->it_pending + 1;
+  const bool last = it >= st->maxit;
+  const bool done = broken || met || last;
+  if (blockIdx.x == 0 && threadIdx.x == 0)
+  {
+    st->rz_next = v[0];
+    st->rr = v[1];
+    st->it = it;
+    if (done)
+    {
+      st->status = broken ? FEMTC_ERR_BREAKDOWN
+                   : met  ? FEMTC_OK
+                          : FEMTC_ERR_NOT_CONVERGED;
+      st->done = 1;
+    }
+  }
+  if (done)
   {
     GRID_LOOP(i, n) { e[i] += a * p[i]; }
     return;
   }
-  const V b = (V)st->beta;
+  const V b = (V)(v[0] / rz);
   GRID_LOOP(i, n)
   {
     const V pi = p[i];
@@ -383,10 +432,10 @@ __global__ void __launch_bounds__(RB)
 }
 
 __global__ void __launch_bounds__(RB)
-    k_combine1(const double* __restrict__ part, double* out)
+    k_combine1(const double* __restrict__ part, int npart, double* out)
 {
   double v[1];
-  combine_partials<1>(part, v);
+  combine_partials<1>(part, npart, v);
   if (threadIdx.x == 0)
     *out = v[0];
 }
@@ -620,6 +669,9 @@ struct femtc_solver
   double* r64 = nullptr;
   double* Au64 = nullptr;
   double* part = nullptr;
+  double* epart2 = nullptr; // block partials of the operator's energies
+  int nblk = 1;             // blocks of the vector kernels
+  int npart = 1;            // partials the last update launch writes
   double* dscal = nullptr; // device scalar for norms
   int* dbad = nullptr;
   PcgState* st = nullptr;
@@ -712,6 +764,7 @@ void destroy(femtc_solver* S)
   dev_free(S->r64);
   dev_free(S->Au64);
   dev_free(S->part);
+  dev_free(S->epart2);
   dev_free(S->dscal);
   dev_free(S->dbad);
   dev_free(S->st);
@@ -872,19 +925,30 @@ LatticeGrid lattice_grid(const femtc_solver* S)
 template <typename V>
 int launch_update(femtc_solver* S, hipStream_t s)
 {
+  const bool direct = S->nepart <= EPART_DIRECT;
+  const double* energy = direct ? S->epart : S->epart2;
+  const int nenergy =
+      direct ? (int)S->nepart : std::min(S->nblk, vec_blocks(S->nepart));
+  if (!direct)
+    hipLaunchKernelGGL(k_energy_partials, dim3(nenergy), dim3(RB), 0, s,
+                       (const double*)S->epart, S->nepart, S->epart2,
+                       (const PcgState*)S->st);
   if (S->inner_assembled)
   {
     const V* W = (const V*)S->lattice;
     V* r = (V*)S->r;
     const auto* dinv = (const typename Precond<V>::T*)S->dinv;
     const LatticeGrid L = lattice_grid(S);
-    const PcgState* st = S->st;
+    // a row per wave; the p-update combines one partial per block
+    const int nb = (int)std::min<int64_t>(
+        S->nblk, (lattice_global_rows(L) + ARB / 64 - 1) / (ARB / 64));
+    S->npart = nb;
     switch (L.P)
     {
 #define FEMTC_ASM_UPDATE(PP)                                                  \
   case PP:                                                                    \
-    hipLaunchKernelGGL((k_assemble_update<V, PP>), dim3(NBLK), dim3(ARB), 0, \
-                       s, W, r, dinv, L, st, S->part);                        \
+    hipLaunchKernelGGL((k_assemble_update<V, PP>), dim3(nb), dim3(ARB), 0,   \
+                       s, W, r, dinv, L, energy, nenergy, S->st, S->part);    \
     break;
       FEMTC_ASM_UPDATE(1)
       FEMTC_ASM_UPDATE(2)
@@ -900,10 +964,12 @@ int launch_update(femtc_solver* S, hipStream_t s)
     }
   }
   else
-    hipLaunchKernelGGL(k_update<V>, dim3(NBLK), dim3(RB), 0, s, (V*)S->r,
+  {
+    S->npart = S->nblk;
+    hipLaunchKernelGGL(k_update<V>, dim3(S->nblk), dim3(RB), 0, s, (V*)S->r,
                        (V*)S->Ap, (const typename Precond<V>::T*)S->dinv,
-                       S->n,
-                       (const PcgState*)S->st, S->part);
+                       S->n, energy, nenergy, S->st, S->part);
+  }
   return hip_status(hipGetLastError());
 }
 
@@ -1035,8 +1101,14 @@ int choose_variant(femtc_solver* S, int structured)
       if (st == FEMTC_OK)
         st = fill_zero(v, S->n, dt, s);
     PcgState h{};
+    // the update's alpha = r.z / p.Ap must come out as 0: r.z is, and one
+    // positive energy keeps p.Ap from being
+    if (st == FEMTC_OK)
+      st = fill_zero(S->epart, S->nepart_cap, FEMTC_F64, s);
     if (st == FEMTC_OK &&
-        (hipMemcpyAsync(S->st, &h, sizeof(h), hipMemcpyHostToDevice, s) !=
+        (hipMemcpyAsync(S->epart, S->dinv64, 8, hipMemcpyDeviceToDevice, s) !=
+             hipSuccess ||
+         hipMemcpyAsync(S->st, &h, sizeof(h), hipMemcpyHostToDevice, s) !=
              hipSuccess ||
          hipStreamSynchronize(s) != hipSuccess))
       st = fail(FEMTC_ERR_HIP, "solver: state upload failed");
@@ -1119,7 +1191,7 @@ int sync_write(femtc_solver* S, void* dev, const void* host, size_t bytes)
   } while (0)
 
 // check_every CG iterations in precision V, queued on stream s: operator
-// (with the p.Ap energies), alpha, update, beta, p-update.  Every kernel
+// (with the p.Ap energies), update (with alpha), p-update (with beta).  Every kernel
 // returns at once after the state's `done` is set.
 template <typename V>
 int enqueue_batch(femtc_solver* S, hipStream_t s)
@@ -1133,19 +1205,12 @@ int enqueue_batch(femtc_solver* S, hipStream_t s)
     int st = run_inner(S, a);
     if (st != FEMTC_OK)
       return st;
-    hipLaunchKernelGGL(k_energy_partials, dim3(NBLK), dim3(RB), 0, s,
-                       (const double*)S->epart, S->nepart, S->part,
-                       (const PcgState*)S->st);
-    hipLaunchKernelGGL(k_alpha, dim3(1), dim3(RB), 0, s,
-                       (const double*)S->part, S->st);
     if ((st = launch_update<V>(S, s)) != FEMTC_OK)
       return st;
-    hipLaunchKernelGGL(k_beta, dim3(1), dim3(RB), 0, s,
-                       (const double*)S->part, S->st);
-    hipLaunchKernelGGL(k_pupdate<V>, dim3(NBLK), dim3(RB), 0, s, (V*)S->p,
+    hipLaunchKernelGGL(k_pupdate<V>, dim3(S->nblk), dim3(RB), 0, s, (V*)S->p,
                        (V*)S->e, (const V*)S->r,
                        (const typename Precond<V>::T*)S->dinv, S->n,
-                       (const PcgState*)S->st);
+                       (const double*)S->part, S->npart, S->st);
   }
   return hip_status(hipGetLastError());
 }
@@ -1201,11 +1266,11 @@ int pcg_run(femtc_solver* S, double rtol, int maxit, int* iters, int* status)
 {
   hipStream_t s = S->stream;
   const int64_t n = S->n;
-  hipLaunchKernelGGL(k_start<V>, dim3(NBLK), dim3(RB), 0, s, (const V*)S->rhs,
+  hipLaunchKernelGGL(k_start<V>, dim3(S->nblk), dim3(RB), 0, s, (const V*)S->rhs,
                      (V*)S->e, (V*)S->r, (V*)S->p, (V*)S->Ap,
                      (const typename Precond<V>::T*)S->dinv, n, S->part);
   hipLaunchKernelGGL(k_reduce_start, dim3(1), dim3(RB), 0, s,
-                     (const double*)S->part, S->st, rtol, maxit);
+                     (const double*)S->part, S->nblk, S->st, rtol, maxit);
   LAUNCH_CHECK();
   for (;;)
   {
@@ -1235,10 +1300,10 @@ int true_residual(femtc_solver* S, const double* f, const double* u,
   st = run(a);
   if (st != FEMTC_OK)
     return st;
-  hipLaunchKernelGGL(k_residual, dim3(NBLK), dim3(RB), 0, s, f,
+  hipLaunchKernelGGL(k_residual, dim3(S->nblk), dim3(RB), 0, s, f,
                      (const double*)S->Au64, S->r64, S->n, S->part);
   hipLaunchKernelGGL(k_combine1, dim3(1), dim3(RB), 0, s,
-                     (const double*)S->part, S->dscal);
+                     (const double*)S->part, S->nblk, S->dscal);
   LAUNCH_CHECK();
   st = sync_read(S, S->hscal, S->dscal, sizeof(double));
   if (st != FEMTC_OK)
@@ -1249,10 +1314,10 @@ int true_residual(femtc_solver* S, const double* f, const double* u,
 
 int norm2(femtc_solver* S, const double* x, double* out)
 {
-  hipLaunchKernelGGL(k_norm2, dim3(NBLK), dim3(RB), 0, S->stream, x, S->n,
+  hipLaunchKernelGGL(k_norm2, dim3(S->nblk), dim3(RB), 0, S->stream, x, S->n,
                      S->part);
   hipLaunchKernelGGL(k_combine1, dim3(1), dim3(RB), 0, S->stream,
-                     (const double*)S->part, S->dscal);
+                     (const double*)S->part, S->nblk, S->dscal);
   LAUNCH_CHECK();
   int st = sync_read(S, S->hscal, S->dscal, sizeof(double));
   if (st != FEMTC_OK)
@@ -1361,6 +1426,7 @@ int femtc_solver_create(femtc_solver** out, const femtc_problem* prob,
   S->N = prob->degree + 1;
   S->Q = prob->nq;
   S->n = prob->ndofs;
+  S->nblk = vec_blocks(S->n);
   S->stream = (hipStream_t)stream;
   const int64_t n = S->n;
   const int64_t C = prob->num_cells;
@@ -1374,6 +1440,7 @@ int femtc_solver_create(femtc_solver** out, const femtc_problem* prob,
         (st = dev_alloc(S, (void**)&S->r64, 8 * n)) ||
         (st = dev_alloc(S, (void**)&S->Au64, 8 * n)) ||
         (st = dev_alloc(S, (void**)&S->part, 8 * 2 * NBLK)) ||
+        (st = dev_alloc(S, (void**)&S->epart2, 8 * NBLK)) ||
         (st = dev_alloc(S, (void**)&S->dscal, 8)) ||
         (st = dev_alloc(S, (void**)&S->dbad, sizeof(int))) ||
         (st = dev_alloc(S, (void**)&S->st, sizeof(PcgState))) ||
@@ -1445,7 +1512,7 @@ int femtc_solver_create(femtc_solver** out, const femtc_problem* prob,
       break;
     if ((st = fill_zero(S->dbad, 1, FEMTC_F32, s)) != FEMTC_OK)
       break;
-    hipLaunchKernelGGL(k_invert, dim3(NBLK), dim3(RB), 0, s,
+    hipLaunchKernelGGL(k_invert, dim3(S->nblk), dim3(RB), 0, s,
                        (const double*)S->diag, S->dinv64, n, S->dbad);
     if (inner_dtype == FEMTC_F64)
     {
@@ -1462,12 +1529,12 @@ int femtc_solver_create(femtc_solver** out, const femtc_problem* prob,
           (st = dev_alloc(S, &S->tab, 4 * (ntab + S->Q))) ||
           (st = dev_alloc(S, &S->G, 4 * CELLGEO * C)))
         break;
-      hipLaunchKernelGGL(k_precond_bf16, dim3(NBLK), dim3(RB), 0, s,
+      hipLaunchKernelGGL(k_precond_bf16, dim3(S->nblk), dim3(RB), 0, s,
                          (const double*)S->dinv64, (uint16_t*)S->dinv, n);
-      hipLaunchKernelGGL((k_convert<double, float>), dim3(NBLK), dim3(RB), 0,
+      hipLaunchKernelGGL((k_convert<double, float>), dim3(S->nblk), dim3(RB), 0,
                          s, (const double*)S->tabw64, (float*)S->tab,
                          ntab + S->Q);
-      hipLaunchKernelGGL((k_convert<double, float>), dim3(NBLK), dim3(RB), 0,
+      hipLaunchKernelGGL((k_convert<double, float>), dim3(S->nblk), dim3(RB), 0,
                          s, (const double*)S->cg64, (float*)S->G,
                          (int64_t)CELLGEO * C);
     }
@@ -1476,23 +1543,23 @@ int femtc_solver_create(femtc_solver** out, const femtc_problem* prob,
       if ((st = dev_alloc(S, &S->r, 4 * n)) || (st = dev_alloc(S, &S->dinv, 2 * n)) ||
           (st = dev_alloc(S, &S->tab, 4 * 2 * S->N * S->Q)))
         break;
-      hipLaunchKernelGGL(k_precond_bf16, dim3(NBLK), dim3(RB), 0, s,
+      hipLaunchKernelGGL(k_precond_bf16, dim3(S->nblk), dim3(RB), 0, s,
                          (const double*)S->dinv64, (uint16_t*)S->dinv, n);
-      hipLaunchKernelGGL((k_convert<double, float>), dim3(NBLK), dim3(RB), 0,
+      hipLaunchKernelGGL((k_convert<double, float>), dim3(S->nblk), dim3(RB), 0,
                          s, prob->tables, (float*)S->tab,
                          (int64_t)2 * S->N * S->Q);
       if (prob->G)
       {
         if ((st = dev_alloc(S, &S->G, 4 * 6 * Q3 * C)))
           break;
-        hipLaunchKernelGGL((k_convert<double, float>), dim3(NBLK), dim3(RB),
+        hipLaunchKernelGGL((k_convert<double, float>), dim3(S->nblk), dim3(RB),
                            0, s, prob->G, (float*)S->G, 6 * Q3 * C);
       }
       if (prob->detJw)
       {
         if ((st = dev_alloc(S, &S->detJw, 4 * Q3 * C)))
           break;
-        hipLaunchKernelGGL((k_convert<double, float>), dim3(NBLK), dim3(RB),
+        hipLaunchKernelGGL((k_convert<double, float>), dim3(S->nblk), dim3(RB),
                            0, s, prob->detJw, (float*)S->detJw, Q3 * C);
       }
     }
@@ -1693,7 +1760,7 @@ int femtc_solver_solve(femtc_solver* S, const double* f, double* u,
         break;
       }
       // inner: A_32 e = r / ||r||
-      hipLaunchKernelGGL(k_scale_to<float>, dim3(NBLK), dim3(RB), 0, s,
+      hipLaunchKernelGGL(k_scale_to<float>, dim3(S->nblk), dim3(RB), 0, s,
                          (const double*)S->r64, 1.0 / rn, (float*)S->rhs, n);
       LAUNCH_CHECK();
       // the last step only has to close the remaining gap to rtol: solve
@@ -1711,7 +1778,7 @@ int femtc_solver_solve(femtc_solver* S, const double* f, double* u,
         inf.status = pst;
         break;
       }
-      hipLaunchKernelGGL(k_correct<float>, dim3(NBLK), dim3(RB), 0, s, u,
+      hipLaunchKernelGGL(k_correct<float>, dim3(S->nblk), dim3(RB), 0, s, u,
                          (const float*)S->e, rn, n);
       LAUNCH_CHECK();
       double rn_new = 0.0;
