@@ -51,13 +51,30 @@ def _ptr(a):
     raise TypeError(f"expected a device tensor, got {type(a)}")
 
 
+def _current_stream():
+    """The handle of torch's current stream on its current device.
+
+    torch.cuda.current_stream() builds a Stream object (2.9 us, a third of a
+    small apply's call); the handle alone takes 0.2 us where torch offers it,
+    once it has initialised the device."""
+    try:
+        import torch
+    except Exception:  # torch absent: default stream
+        return None
+    if torch.cuda.is_initialized():
+        try:
+            return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+        except AttributeError:
+            pass
+    try:
+        return torch.cuda.current_stream().cuda_stream
+    except Exception:  # no device: default stream
+        return None
+
+
 def _stream(stream):
     if stream is None:
-        try:
-            import torch
-            return torch.cuda.current_stream().cuda_stream
-        except Exception:  # torch absent or no device: default stream
-            return None
+        return _current_stream()
     if isinstance(stream, int):
         return stream
     return stream.cuda_stream
