@@ -33,6 +33,7 @@
 #include <algorithm>
 #include <utility>
 
+#include "cell_common.hpp"
 #include "common.hpp"
 
 namespace femtc
@@ -74,21 +75,6 @@ constexpr int line_base_op(int op)
   return op >= OP_MASS_AFF ? op - OP_MASS_AFF : op;
 }
 
-// Waves per SIMD a cell's registers are sized for: 3 (168 VGPRs), or 2
-// (256 VGPRs) for FP64 stiffness and K+M when the values live at once --
-// the three gradient lines (and u) at Q points plus one line of N -- do not
-// fit 168 without spilling (bounds from the compiler's counts over the
-// instantiated shapes).
-template <typename T, int OP, int N, int Q>
-constexpr int line_want()
-{
-  constexpr bool f64 = sizeof(T) == 8;
-  constexpr int B = line_base_op(OP);
-  return (f64 && B == OP_STIFF && 3 * Q + N > LINE_STIFF64_LIVE)  ? 2
-         : (f64 && B == OP_KPM && 4 * Q + N > LINE_KPM64_LIVE) ? 2
-                                                                : 3;
-}
-
 // LDS slices per cell: two alternating slices (one barrier per transpose)
 // when they fit the 160 KB of a CU, else one (two barriers per transpose).
 template <typename T, int N, int Q>
@@ -103,6 +89,25 @@ template <typename T, int N, int Q>
 constexpr size_t line_cell_lds()
 {
   return line_nbuf<T, N, Q>() * (size_t)LineShape<N, Q>::SLICE * sizeof(T);
+}
+
+// Waves per SIMD a cell's registers are sized for: 3 (168 VGPRs), or 2
+// (256 VGPRs) for FP64 stiffness and K+M when the values live at once --
+// the three gradient lines (and u) at Q points plus one line of N -- do not
+// fit 168 without spilling (bounds from the compiler's counts over the
+// instantiated shapes), or when the LDS of cells of 4 waves keeps two of
+// them on a CU, so that a third wave per SIMD cannot become resident.
+template <typename T, int OP, int N, int Q>
+constexpr int line_want()
+{
+  constexpr bool f64 = sizeof(T) == 8;
+  constexpr int B = line_base_op(OP);
+  return (f64 && B == OP_STIFF && 3 * Q + N > LINE_STIFF64_LIVE)  ? 2
+         : (f64 && B == OP_KPM && 4 * Q + N > LINE_KPM64_LIVE) ? 2
+         : (f64 && LineShape<N, Q>::TH <= 256 &&
+            3 * line_cell_lds<T, N, Q>() > 160 * 1024)
+             ? 2
+             : 3;
 }
 
 // Registers a cell's values need: the values live at once (mass: a line of
@@ -312,10 +317,76 @@ __device__ __forceinline__ void line_bwd(const T* M, const T (&in)[NI],
   line_contract<T, NI, NO, true, ACC>(M, in, out);
 }
 
+// The staged geometry's split: CH points of every line are one chunk of PL
+// two-value pieces per line.  Thread t of a cell takes piece t % PL of lines
+// t / PL + i LP, i < PASS: the addresses of a thread's pieces then differ by
+// amounts that are the same for all threads and need one register (and one
+// for the last pass, whose lines are clamped).
+template <int N, int Q, int CH_>
+struct LineStage
+{
+  using S = LineShape<N, Q>;
+  static constexpr int CH = CH_;
+  static constexpr int PL = 3 * CH;
+  static constexpr int LP = S::TH / PL;
+  static constexpr int PASS = (S::QQ + LP - 1) / LP;
+  static constexpr int BUF = PASS * LP * PL; // pieces of one buffer
+  static constexpr int NCH = (Q + CH - 1) / CH;
+};
+
+// Whether the geometry of a stiffness or K+M cell is staged through LDS:
+// wherever two chunks of two points fit the cell's slices (N >= 14, and
+// N >= 12 at Q = N + 2), up to 4 Q + N = 118 for FP32 K+M.  Measured on 20 M
+// dofs against reading it by the line with the next point in flight: FP64
+// stiffness N=14 1.20x, N=16 1.24x, N=17 1.16x, N=18 1.00x, N=20 1.08x, K+M
+// N=16 1.36x; FP32 stiffness N=14..21 1.17-1.32x; against the deepest
+// prefetch that fits the registers (line_geo_depth) 1.0-1.25x.  FP32 K+M
+// N=24 spills: 0.98x, by the line 1.07x.
+template <typename T, int OP, int N, int Q>
+constexpr bool line_staged()
+{
+  return (OP == OP_STIFF ||
+          (OP == OP_KPM && (sizeof(T) == 8 || 4 * Q + N <= 118))) &&
+         2 * LineStage<N, Q, 2>::BUF * sizeof(Piece<T>) <=
+             line_cell_lds<T, N, Q>();
+}
+
+// Barriers the second cell of a staged two-cell workgroup stays behind the
+// first: half of a cell's barriers (10 transposes, one per chunk, two around
+// them), so that one cell streams its geometry while the other contracts.
+template <typename T, int OP, int N, int Q>
+constexpr int line_skew()
+{
+  return line_cpb<T, OP, N, Q>() == 2 && line_staged<T, OP, N, Q>()
+             ? (12 + LineStage<N, Q, 2>::NCH) / 2
+             : 0;
+}
+
+// Points of geometry in flight where it is read by the line: as many as the
+// registers left by the cell's values hold, 1 to 5 (mass, one value a point:
+// 5; affine cells compute theirs).  Against one point, 20 M dofs: FP64
+// stiffness N=10 1.12x, N=13 1.05x, FP32 N=10 1.29x, N=13 1.26x, FP64 mass
+// N=10 1.05x, N=17 1.12x.  One point more than fits spills: FP64 K+M N=12,
+// Q=13 at two points 0.95x.
+template <typename T, int OP, int N, int Q>
+constexpr int line_geo_depth()
+{
+  constexpr int B = line_base_op(OP);
+  if (OP >= OP_MASS_AFF)
+    return 1;
+  if (B == OP_MASS)
+    return 5;
+  constexpr int per = (B == OP_STIFF ? 6 : 7) * (int)(sizeof(T) / 4);
+  constexpr int d = (line_budget(line_waves<T, OP, N, Q>()) -
+                     line_vgprs<T, OP, N, Q>() + 4) /
+                    per;
+  return d < 1 ? 1 : d > 5 ? 5 : d;
+}
+
 // The quadrature-point stage of owner (qa,qb) = tq on its Q points
 // (qa,qb,qc): (d_a, d_b, d_c) <- S(q) (d_a, d_b, d_c) with
 // S = [[G5,G4,G2],[G4,G3,G1],[G2,G1,G0]] (stiffness), u <- detJw u (mass),
-// one point at a time with the next point's geometry in flight.
+// one point at a time with the geometry of the next ones in flight.
 template <typename T, int OP, int N, int Q, int NA, int NU>
 __device__ __forceinline__ void line_pointwise(const T* __restrict__ G,
                                                const T* __restrict__ detJw,
@@ -344,7 +415,6 @@ __device__ __forceinline__ void line_pointwise(const T* __restrict__ G,
     const int qa = tq / Q;
     wab = wts[qa] * wts[tq - qa * Q];
   }
-  T gcur[GV], gnxt[GV];
   auto load = [&](int qc, T (&gb)[GV]) {
     if constexpr (AFF)
     {
@@ -371,32 +441,137 @@ __device__ __forceinline__ void line_pointwise(const T* __restrict__ G,
         gb[GV - 1] = detJw[p0 + qc];
     }
   };
-  load(0, gcur);
+  constexpr int D = line_geo_depth<T, OP, N, Q>();
+  static_assert(D <= Q, "points to load ahead");
+  T ring[D + 1][GV];
+  line_static_for<D>([&](auto qcc) {
+    constexpr int qc = decltype(qcc)::value;
+    load(qc, ring[qc]);
+  });
   line_static_for<Q>([&](auto qcc) {
     constexpr int qc = decltype(qcc)::value;
     __builtin_amdgcn_sched_barrier(0);
-    if constexpr (qc + 1 < Q)
-      load(qc + 1, gnxt);
+    if constexpr (qc + D < Q)
+      load(qc + D, ring[(qc + D) % (D + 1)]);
+    const T(&g)[GV] = ring[qc % (D + 1)];
     if constexpr (FULL)
     {
       const T da = DA[qc], db = DB[qc], dcv = DC[qc];
-      DA[qc] = gcur[5] * da + gcur[4] * db + gcur[2] * dcv;
-      DB[qc] = gcur[4] * da + gcur[3] * db + gcur[1] * dcv;
-      DC[qc] = gcur[2] * da + gcur[1] * db + gcur[0] * dcv;
+      DA[qc] = g[5] * da + g[4] * db + g[2] * dcv;
+      DB[qc] = g[4] * da + g[3] * db + g[1] * dcv;
+      DC[qc] = g[2] * da + g[1] * db + g[0] * dcv;
       asm volatile("" : "+v"(DA[qc]), "+v"(DB[qc]), "+v"(DC[qc]));
     }
     if constexpr (MT)
     {
-      U[qc] *= gcur[GV - 1];
+      U[qc] *= g[GV - 1];
       asm volatile("" : "+v"(U[qc]));
     }
-    if constexpr (qc + 1 < Q)
+  });
+}
+
+// The same stage with the geometry staged through the cell's idle LDS slices
+// (buf).  A thread's own line is 6 Q contiguous values: the loads of a wave
+// by the line touch 64 places 48 Q bytes apart, each cache line of them is
+// wanted again at the next points, and by then the other lines have pushed
+// it out of the L1 (FP64 N=17: 540 us on 20 M dofs by the line, 452 when the
+// same bytes were read in lane order, 325 without them).  Here the threads
+// of the cell read a chunk's pieces lane after lane into registers while
+// they work on the chunk before, write them to LDS and pick their own points
+// from there.  Two buffers alternate: one barrier per chunk orders the reads
+// of a chunk after its writes and the writes two chunks later after those
+// reads.  Two points per chunk: one point doubles the barriers (N=17 508 us
+// against 450), three do not fit the slices; two chunks in flight spill in
+// FP64 and gain nothing in FP32.
+template <typename T, int OP, int N, int Q, int NA, int NU>
+__device__ __forceinline__ void
+line_pointwise_staged(const T* __restrict__ G, const T* __restrict__ detJw,
+                      int64_t cell, int t, int tq, T* buf, T (&DA)[NA],
+                      T (&DB)[NA], T (&DC)[NA], T (&U)[NU])
+{
+  using S = LineShape<N, Q>;
+  constexpr bool MT = OP == OP_KPM;
+  using L = LineStage<N, Q, 2>;
+  constexpr int CH = L::CH, PL = L::PL, PASS = L::PASS, NCH = L::NCH;
+  static_assert(2 * L::BUF * sizeof(Piece<T>) <= line_cell_lds<T, N, Q>(),
+                "two chunks fit the slices");
+  static_assert(line_cell_lds<T, N, Q>() % sizeof(Piece<T>) == 0 ||
+                    line_cpb<T, OP, N, Q>() == 1,
+                "every cell's slices are aligned");
+  const Piece<T>* const Gc =
+      reinterpret_cast<const Piece<T>*>(G + cell * (int64_t)(6 * Q * Q * Q));
+  const T* const dc = MT ? detJw + cell * (int64_t)(Q * Q * Q) : nullptr;
+  // threads past the last whole line repeat the last one's piece, lines past
+  // the last repeat the last line
+  const int tp = t < L::LP * PL ? t : L::LP * PL - 1;
+  const int ln = tp / PL, j0 = tp - ln * PL;
+  constexpr int LAST = S::QQ - 1 - (PASS - 1) * L::LP;
+  const int off = ln * 3 * Q + j0;
+  const int offl = (ln < LAST ? ln : LAST) * 3 * Q + j0;
+  Piece<T>* const B = reinterpret_cast<Piece<T>*>(buf) + tp;
+  const Piece<T>* const R = reinterpret_cast<Piece<T>*>(buf) + tq * PL;
+  Piece<T> g[PASS];
+  T dw[CH];
+  auto load = [&](int k) {
+#pragma unroll
+    for (int i = 0; i < PASS; ++i)
+    {
+      int o = i + 1 < PASS ? off : offl;
+      // a last chunk that is not full reads the next line's first values;
+      // the last line's stay on its last piece
+      if ((k + 1) * CH > Q && i + 1 == PASS)
+      {
+        const int last = LAST * 3 * Q + 3 * Q - 1 - k * PL;
+        o = o < last ? o : last;
+      }
+      g[i] = (Gc + (i * L::LP * 3 * Q + k * PL))[(unsigned)o];
+    }
+    if constexpr (MT)
     {
 #pragma unroll
-      for (int k = 0; k < GV; ++k)
-        gcur[k] = gnxt[k];
+      for (int j = 0; j < CH; ++j)
+        dw[j] =
+            (dc + (k * CH + j < Q ? k * CH + j : Q - 1))[(unsigned)(tq * Q)];
     }
+  };
+  load(0);
+  lds_barrier(); // the slices' last transpose has been read
+  line_static_for<NCH>([&](auto kc) {
+    constexpr int k = decltype(kc)::value;
+#pragma unroll
+    for (int i = 0; i < PASS; ++i)
+      B[(k & 1) * L::BUF + i * L::LP * PL] = g[i];
+    T d[CH];
+    if constexpr (MT)
+    {
+#pragma unroll
+      for (int j = 0; j < CH; ++j)
+        d[j] = dw[j];
+    }
+    if constexpr (k + 1 < NCH)
+      load(k + 1);
+    lds_barrier();
+    line_static_for<CH>([&](auto jc) {
+      constexpr int j = decltype(jc)::value;
+      constexpr int qc = k * CH + j;
+      if constexpr (qc < Q)
+      {
+        const Piece<T>* const r = R + (k & 1) * L::BUF + 3 * j;
+        const Piece<T> p0 = r[0], p1 = r[1], p2 = r[2];
+        const T da = DA[qc], db = DB[qc], dcv = DC[qc];
+        DA[qc] = p2.y * da + p2.x * db + p1.x * dcv;
+        DB[qc] = p2.x * da + p1.y * db + p0.y * dcv;
+        DC[qc] = p1.x * da + p0.y * db + p0.x * dcv;
+        asm volatile("" : "+v"(DA[qc]), "+v"(DB[qc]), "+v"(DC[qc]));
+        if constexpr (MT)
+        {
+          U[qc] *= d[j];
+          asm volatile("" : "+v"(U[qc]));
+        }
+      }
+    });
   });
+  lds_barrier(); // the chunks are read; the slices may be rewritten
 }
 
 template <typename T, int OP, int N, int Q>
@@ -427,6 +602,26 @@ __global__ void __launch_bounds__((line_threads<T, OP, N, Q>()))
   const T* const phi = tab; // [dof][q]
   const T* const dph = tab + N * Q;
 
+  // The two cells of a staged workgroup run SKEW barriers apart where the
+  // workgroup takes several pairs: the second cell's waves wait at SKEW extra
+  // barriers before their first cell, the first cell's at as many after
+  // their last, so every wave arrives at the same number.  The cells share
+  // no LDS; the waves of one cell stay in step.
+  constexpr int SKEW = line_skew<T, OP, N, Q>();
+  const bool skewed = C > (int64_t)gridDim.x * CPB;
+  auto skew = [&](bool second) {
+    if constexpr (SKEW > 0)
+    {
+      if (skewed &&
+          (__builtin_amdgcn_readfirstlane(threadIdx.x) >= S::TH) == second)
+      {
+#pragma unroll 1
+        for (int i = 0; i < SKEW; ++i)
+          __builtin_amdgcn_s_barrier();
+      }
+    }
+  };
+  skew(true);
   for (int64_t c0 = (int64_t)blockIdx.x * CPB; c0 < C;
        c0 += (int64_t)gridDim.x * CPB)
   {
@@ -636,7 +831,11 @@ __global__ void __launch_bounds__((line_threads<T, OP, N, Q>()))
       __syncthreads();
       r_ab_c(4, l);
       line_fwd<T, N, Q>(phi, l, DA);
-      line_pointwise<T, OP, N, Q>(G, detJw, tab, cell, tab_, DA, DB, DC, U);
+      if constexpr (line_staged<T, OP, N, Q>())
+        line_pointwise_staged<T, OP, N, Q>(G, detJw, cell, t, tab_, slice0, DA,
+                                           DB, DC, U);
+      else
+        line_pointwise<T, OP, N, Q>(G, detJw, tab, cell, tab_, DA, DB, DC, U);
       // B_c along c, each result to LDS as soon as it is complete
       T D1[N], D2[N], D3[N];
       line_bwd<T, Q, N>(dph, DC, D3);
@@ -722,6 +921,7 @@ __global__ void __launch_bounds__((line_threads<T, OP, N, Q>()))
       }
     }
   }
+  skew(false);
 }
 
 // Launch for one (N, Q): the op and dtype from the request.
@@ -732,8 +932,22 @@ int line_launch_op(const ApplyReq& r, int max_lds)
   if (bytes > (size_t)max_lds)
     return FEMTC_ERR_INVALID_ARGUMENT;
   constexpr int CPB = line_cpb<T, OP, N, Q>();
-  const int64_t grid64 =
-      std::min<int64_t>((r.num_cells + CPB - 1) / CPB, 16384);
+  int64_t grid64 = std::min<int64_t>((r.num_cells + CPB - 1) / CPB, 16384);
+  if constexpr (line_skew<T, OP, N, Q>() > 0)
+  {
+    // One workgroup of two staged cells is resident on a CU (10 waves or
+    // more, over 96 VGPRs).  From four pairs per CU on, one workgroup per CU
+    // takes all of them with its cells a half apart; fewer pairs do not make
+    // up for the half cell at either end.  20 M dofs, in step / a half
+    // apart: FP64 stiffness N=17 519 / 448 us; FP32 stiffness N=17 374 / 351,
+    // K+M 469 / 390.
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) == hipSuccess &&
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount,
+                              dev) == hipSuccess &&
+        cus > 0 && grid64 >= 4 * (int64_t)cus)
+      grid64 = cus;
+  }
   hipLaunchKernelGGL((line_cells<T, OP, N, Q>), dim3((unsigned)grid64),
                      dim3(line_threads<T, OP, N, Q>()), bytes, r.stream,
                      (const T*)r.tab, (const T*)r.x, (T*)r.y, (const T*)r.G,
