@@ -81,11 +81,33 @@ constexpr int block_threads()
   return ((cells_per_block<Q>() * Q * Q + 63) / 64) * 64;
 }
 
+// Cells of a cell-local workgroup that packs them over 4 waves.
+constexpr int LOCAL_PACK = 7;
+
+// Fewest cells from which a cell-local apply packs its workgroups (0: never).
+// At Q = 6 one cell in a wave keeps 36 of its 64 lanes busy, 7 cells in 4
+// waves 252 of 256.  With few cells a wave's own latency sets the time, and
+// the barriers of 4 waves add to it.  One cell per wave against 7 in four, us
+// on MI355X: FP64 mass P=5 50 cells 3.4 / 4.0, 1500 4.3 / 4.5, 6000 8.4 / 8.1,
+// 92,592 99.3 / 92.6; FP32 mass P=3 1500 cells 3.2 / 3.1, 312,500 119 / 82;
+// FP32 stiffness P=5 300 cells 5.1 / 6.7, 6000 12.7 / 13.0, 40,000 58.7 / 54.6,
+// 92,592 132 / 120.  FP64 gradient operators measured the same either way, and
+// at Q = 5 and 7 (50 and 49 of 64 lanes) 10 and 5 cells in 4 waves were mixed.
+template <typename T, int OP, int Q>
+constexpr int local_pack_cells()
+{
+  return Q != 6                ? 0
+         : OP == OP_MASS       ? 4096
+         : sizeof(T) == 4 && (OP == OP_STIFF || OP == OP_KPM) ? 32768
+                                                              : 0;
+}
+
 // Cells and threads per workgroup of an instance with scatter kind BW.
 template <typename T, int Q, int BW>
 constexpr int cells_per_group()
 {
   return BW == SCATTER_ASSEMBLED ? assembled_cells(Q, (int)sizeof(T))
+         : BW == SCATTER_LOCAL   ? LOCAL_PACK
                                  : cells_per_block<Q>();
 }
 
@@ -1414,10 +1436,16 @@ int launch_batch_n(const BatchReq& r)
 
 // Launch one instance: one workgroup per batch of CPB cells.
 template <typename T, int N, int Q, int OP, bool REF, bool GATHER,
-          bool EO = false>
+          bool EO = false, int BW = 0>
 int launch_cells(const ApplyReq& r)
 {
-  constexpr int CPB = cells_per_block<Q>();
+  // cell-local applies of many cells at Q = 6
+  if constexpr (BW == 0 && !GATHER && !REF && local_pack_cells<T, OP, Q>() > 0)
+  {
+    if (r.num_cells >= local_pack_cells<T, OP, Q>())
+      return launch_cells<T, N, Q, OP, REF, GATHER, EO, SCATTER_LOCAL>(r);
+  }
+  constexpr int CPB = cells_per_group<T, Q, BW>();
   constexpr long long XC = xcd_chunk<T, Q, GATHER>();
   const long long nblk = (r.num_cells + CPB - 1) / CPB;
   if (nblk == 0)
@@ -1428,8 +1456,8 @@ int launch_cells(const ApplyReq& r)
   ba.nblk = (int)nblk;
   const long long grid =
       XC > 1 ? 8 * XC * ((nblk + 8 * XC - 1) / (8 * XC)) : nblk;
-  hipLaunchKernelGGL((apply_cells<T, N, Q, OP, REF, GATHER, 0, EO>),
-                     dim3((unsigned)grid), dim3(block_threads<Q>()), 0,
+  hipLaunchKernelGGL((apply_cells<T, N, Q, OP, REF, GATHER, BW, EO>),
+                     dim3((unsigned)grid), dim3(group_threads<T, Q, BW>()), 0,
                      r.stream, (const T*)(EO ? r.eo_tab : r.tab),
                      (const T*)r.x, (T*)r.y,
                      (const T*)r.G, (const T*)r.detJw, r.dofmap,

@@ -94,6 +94,9 @@ constexpr int SCATTER_ASSEMBLED = -1;
 constexpr int SCATTER_STRUCT = -2;
 // BW template value of the structured z-run scatter (ApplyReq::zrun).
 constexpr int SCATTER_ZRUN = -3;
+// BW template value of the cell-local instances whose workgroups pack cells
+// over several waves (local_pack_cells).
+constexpr int SCATTER_LOCAL = -4;
 
 // Where the chain kernel (apply_chain.hpp) runs a gathered apply instead of
 // the atomic scatter of apply_kernel.hpp: where the N^3 atomics per cell, not
