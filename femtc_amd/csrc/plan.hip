@@ -1,9 +1,9 @@
 // Scatter plans for the continuous operator over a structured cell
-// numbering: the direct atomic scatter, an LDS-assembled scatter over 3-D
+// numbering: the direct scatter of the one-shot apply, an LDS-assembled scatter over 3-D
 // blocks of cells, or the assembled scatter (a cell pass storing every
 // cell-dof value without atomics, then a pass summing each global dof;
 // offered when the dofmap is verified to be the structured numbering at
-// plan creation), chosen per (nq, dtype, op) by default tables or by timing
+// plan creation), chosen per (nq, dtype, op) by a default or by timing
 // the candidates on the caller's own data (femtc_plan_autotune).
 #include <cfloat>
 #include <cstdio>
@@ -116,30 +116,19 @@ std::vector<Shape> candidates(int nq)
 
 int key_of(int nq, int dtype, int op) { return (nq * 4 + dtype) * 4 + op; }
 
-// Default block shape where the blocked scatter measured faster than the
-// direct one on MI355X (structured meshes of 2.4e7-3.6e7 cell-dofs, nq =
-// degree+1); everything else defaults to the direct scatter.  At degree >= 5
-// and for most stiffness cases the one-wave direct kernel wins: its higher
-// occupancy hides more latency than the blocked LDS assembly saves in
-// atomics.
+// Shape of a plan that has not been autotuned: the direct scatter (the chain
+// kernel where chain_pays), except degree 1 FP64 stiffness and K+M, where
+// blocks of 1 x 2 x 16 cells are the faster of the two.  us per apply of
+// structured meshes, blocked against direct, nq = degree + 1: 155^3 cells at
+// P=1 FP64 stiffness 291 / 313, K+M 333 / 363, mass 164 / 138, FP32 stiffness
+// 241 / 194; 78^3 at P=3 FP64 mass 286 / 199, stiffness 422 / 341, FP32
+// stiffness 324 / 183; 62^3 at P=4 FP64 mass 339 / 210, FP32 K+M 374 / 251.
+// At P = 2..4 every blocked shape that was a default measured 1.2-1.9 times
+// the direct scatter's time.
 Shape default_shape(int degree, int nq, int dtype, int op)
 {
-  if (nq != degree + 1)
-    return Shape{0, 0, 0};
-  const bool f32 = dtype == FEMTC_F32;
-  switch (degree)
-  {
-  case 1: return Shape{1, 2, 16};
-  case 2: return op == FEMTC_OP_MASS ? Shape{1, 4, 7} : Shape{0, 0, 0};
-  case 3:
-    if (f32)
-      return Shape{2, 2, 4};
-    return op == FEMTC_OP_KPM ? Shape{0, 0, 0} : Shape{2, 2, 8};
-  case 4:
-    if (op == FEMTC_OP_MASS || f32)
-      return Shape{1, 2, 4};
-    return Shape{0, 0, 0};
-  }
+  if (degree == 1 && nq == 2 && dtype == FEMTC_F64 && op != FEMTC_OP_MASS)
+    return Shape{1, 2, 16};
   return Shape{0, 0, 0};
 }
 

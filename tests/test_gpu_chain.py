@@ -108,3 +108,32 @@ def test_periodic_single_cell():
         check("mass", P, Q, (2, 2, 1), "periodic", torch.float64)
         check("stiffness", P, Q, (2, 2, 1), "periodic", torch.float32,
               affine=True)
+
+
+@pytest.mark.parametrize("kind", ["lex", "reader", "relabelled"])
+@pytest.mark.parametrize("P", [1, 2, 3, 4])
+def test_plan_that_was_not_tuned(P, kind):
+    """A plan's first apply: direct but for degree 1 FP64 stiffness, K+M."""
+    Q, dims = P + 1, (3, 5, 17)
+    dm, ng = numbered(kind, dims, P)
+    C = int(np.prod(dims))
+    G, Dw = O.geometry_affine(O.random_jacobians(5, C), Q)
+    tab, x = O.basis_tables(P, Q), O.uniform(11, ng)
+    y0 = O.uniform(12, ng)
+    plan = F.Plan(*dims, P, torch.from_numpy(dm).cuda(), ng)
+    for op, code in (("mass", F.OP_MASS), ("stiffness", F.OP_STIFFNESS),
+                     ("kpm", F.OP_KPM)):
+        ref = O.global_operator(op, P + 1, Q, tab, x, dm, G, Dw)
+        for dtype, dt in ((torch.float64, F.F64), (torch.float32, F.F32)):
+            blocked = P == 1 and dt == F.F64 and op != "mass"
+            assert plan.get_block(Q, dt, code) == ((1, 2, 16) if blocked
+                                                   else (0, 0, 0))
+            dtab, dx, dG, dD, y = (torch.from_numpy(a).to("cuda", dtype)
+                                   for a in (tab, x, G, Dw, y0))
+            for accumulate in (False, True):
+                plan.apply(code, dtab, dx, y, Q, G=dG, detJw=dD,
+                           accumulate=accumulate)
+            torch.cuda.synchronize()
+            got = y.double().cpu().numpy()
+            err = np.linalg.norm(got - 2 * ref) / np.linalg.norm(2 * ref)
+            assert err <= TOL[dtype], (op, P, kind, dtype, err)
