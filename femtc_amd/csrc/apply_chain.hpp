@@ -28,11 +28,23 @@
 // 256 lanes): affine FP64 K+M at P=5, 97,290 cells, 248 -> 218 us.  At Q = 5
 // and 7 (50 and 49 lanes) the same packing was neutral or slower.
 //
-// Measured (MI355X, overwriting applies with the clear of y, us, the
-// gathered kernel of apply_kernel.hpp against this one): FP32 mass P=3 Q=5,
-// 61x67x71 cells, lexicographic 288 -> 118 and reader order 361 -> 120; FP32
-// stiffness P=4, 64^3, 485 -> 242; affine FP64 K+M P=5, 45x46x47, 288 -> 236;
-// FP64 mass P=7, 40x41x42, 417 -> 301.
+// Where the numbering does not chain (shuffled cells, cells one after another
+// along another axis, plates of one cell) the box would write runs of P and
+// single left-face values where the lanes hold runs of N.  A workgroup
+// therefore looks at its first two pairs of cells, and if neither shares the
+// dof of row (1, 1) every lane adds its values to y as the gathered kernel's
+// do: FP32 mass P=7, local axes rotated, 213 -> 56 us, P=3, shuffled, 196 ->
+// 114.  The dofs wait in the box's place: held in registers they took 1-2
+// waves per SIMD from many shapes.
+//
+// Measured (MI355X, overwriting applies with the clear of y, 3e6 dofs, us, the
+// gathered kernel of apply_kernel.hpp against this one; cells and dofs
+// lexicographic, in reader order, and lexicographic dofs with shuffled cells):
+//   FP32 mass P=3          115 /  42   188 /  55   114 / 114
+//   FP32 stiffness P=4      96 /  54   141 /  55    94 /  90
+//   FP64 mass P=7           66 /  53    89 /  56    70 /  65
+//   affine FP64 K+M P=5     88 /  77   120 /  73    89 / 103
+//   FP32 mass P=1          299 /  87   298 /  87   622 / 620
 #pragma once
 
 #include "cell_chain.hpp"
@@ -80,6 +92,13 @@ struct ChainShape
   static constexpr int LDSW = (WORK + 1) / 2; // pieces per group
   static constexpr size_t LDS = sizeof(Piece<T>) * (size_t)NG * LDSW +
                                 (sizeof(T) + sizeof(int32_t)) * (size_t)BOX;
+  // an unchained workgroup keeps its dofs [b][cell][a][c] in the place of the
+  // box and its dofs, and (PACK) its values in the work area
+  static_assert((size_t)S * N * N * N * sizeof(int32_t) <=
+                    (sizeof(T) + sizeof(int32_t)) * (size_t)BOX,
+                "the dofs fit the box");
+  static_assert(!PACK || S * N * N * N <= 2 * LDSW,
+                "the values fit the work area");
 };
 
 template <typename T, int N, int Q, int OP>
@@ -135,6 +154,18 @@ __global__ void __launch_bounds__((64 * chain_waves<T, Q, OP>()))
   const int yo3 = q3b * Ch::YQ + q3c;
   const bool on1 = live && ln < NN, on2 = live && ln < N * Q;
   const int slot0 = r1a * SA + k * P + r1c;
+
+  // the dofs of row (1, 1) on either side of the chain's first two pairs of
+  // neighbours (scalar loads; a cell alone is compared with itself)
+  int32_t here[2], there[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+  {
+    const int kk = i + 1 < ncell ? i + 1 : ncell - 1;
+    const int32_t* d = dofmap + (chain0 + kk) * N3 + NN + N;
+    here[i] = d[0];
+    there[i] = d[ncell > 1 ? P - N3 : 0];
+  }
 
   // ---------------- loads ----------------------------------------------
   typename Ch::Tab tabs;
@@ -200,12 +231,22 @@ __global__ void __launch_bounds__((64 * chain_waves<T, Q, OP>()))
     for (int q = 0; q < Q; ++q)
       dw[q] = stream_load(Dp + q * Q2);
   }
+  // Whether the numbering chains here.  Looked at only now: a wait for the
+  // scalar loads before the gather of x cost 10 % at P=1.
+  __builtin_amdgcn_sched_barrier(0);
+  const bool chained = here[0] == there[0] || here[1] == there[1];
+  // the line's dofs: to the box's slots, or to the lane's own place
+  int32_t* own = reinterpret_cast<int32_t*>(box) + k * NN + ln1;
+  int32_t* ids = chained ? gid + slot0 : own;
+  const int idstep = chained ? Z : Sh::S * NN;
+  if (!chained)
+    miss = 0;
   if (on1)
   {
 #pragma unroll
     for (int b = 0; b < N; ++b)
       if (!((miss >> b) & 1u))
-        gid[slot0 + b * Z] = idx[b];
+        ids[b * idstep] = idx[b];
   }
 
   // ---------------- the cells' contraction chain ------------------------
@@ -281,6 +322,47 @@ __global__ void __launch_bounds__((64 * chain_waves<T, Q, OP>()))
   Ch::b1(tabs, Xc, r1a, r1c, w);
 
   // ---------------- the chain's box, then y ------------------------------
+  if (!chained)
+  {
+    // nothing to merge: every value from its lane, the N^2 lines of a cell in
+    // one instruction (packed cells straddle the waves and change lanes for
+    // that: FP32 mass P=4, Q=6, local axes rotated, 107 -> 86 us)
+    if constexpr (Sh::PACK)
+    {
+      lds_barrier(); // X is read
+      T* val = reinterpret_cast<T*>(Ls);
+      if (on1)
+      {
+#pragma unroll
+        for (int b = 0; b < N; ++b)
+          val[(b * Sh::S + k) * NN + ln] = w[b];
+      }
+      lds_barrier();
+      const int l = (int)(threadIdx.x & 63);
+      for (int c = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+           c < ncell; c += Sh::BT / 64)
+        if (l < NN)
+        {
+#pragma unroll
+          for (int b = 0; b < N; ++b)
+          {
+            const int o = (b * Sh::S + c) * NN + l;
+            atomic_add(y + reinterpret_cast<int32_t*>(box)[o], val[o]);
+          }
+        }
+    }
+    else if (on1)
+    {
+      int32_t id[N];
+#pragma unroll
+      for (int b = 0; b < N; ++b)
+        id[b] = own[b * (Sh::S * NN)];
+#pragma unroll
+      for (int b = 0; b < N; ++b)
+        atomic_add(y + id[b], w[b]);
+    }
+    return; // uniform over the workgroup
+  }
   if (on1 && !face)
   {
 #pragma unroll

@@ -113,6 +113,11 @@ constexpr int SCATTER_LOCAL = -4;
 //   FP64 stiffness, K+M            1.05-2.3 at Q = N <= 5 (K+M at P=2: 0.94
 //                                  lexicographic, 1.7 in reader order),
 //                                  0.91-1.06 elsewhere
+// Where the numbering does not chain (the kernel then writes as the atomic
+// scatter does; shuffled cells, local axes rotated, reversed lines, 3e6 dofs):
+// 0.94-1.16, but 0.86-0.93 for affine FP64 stiffness and K+M at Q = 6 and
+// 0.88-0.9 for FP32 mass and affine at P = 1, Q = 4; on plates of 1..3 cells
+// 0.9-1.6, but 0.79-0.9 at P = 1, Q = 3 and 4 (1.2-2.6 on cubes).
 // A cell of Q >= 9 does not fit one wave: the chain would be too short.
 constexpr bool chain_pays(int op, bool f64, int N, int Q)
 {

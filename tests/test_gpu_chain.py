@@ -137,3 +137,86 @@ def test_plan_that_was_not_tuned(P, kind):
             got = y.double().cpu().numpy()
             err = np.linalg.norm(got - 2 * ref) / np.linalg.norm(2 * ref)
             assert err <= TOL[dtype], (op, P, kind, dtype, err)
+
+
+def chained_in_part(P, nz, links, seed=3):
+    """(dofmap, number of dofs) of nz cells in a row along z, where cell k
+    (k > 0) shares its left face with cell k-1 only if k is in `links`."""
+    N = P + 1
+    dm = np.empty((nz, N, N, N), dtype=np.int64)
+    n = 0
+    for k in range(nz):
+        first = 0
+        if k in links:
+            dm[k, :, :, 0] = dm[k - 1, :, :, P]
+            first = 1
+        new = N * N * (N - first)
+        dm[k, :, :, first:] = n + np.arange(new).reshape(N, N, N - first)
+        n += new
+    dm = np.random.default_rng(seed).permutation(n)[dm]
+    return np.ascontiguousarray(dm.ravel(), dtype=np.int32), n
+
+
+# the kernel looks at the first two pairs of a chain: merged cells where it
+# takes the whole chain for unmerged, single cells where it merges, and chains
+# of one and two cells (P=5: cells straddling waves)
+LINKS = [set(), {1}, {2}, {3, 4, 6}, {1, 5}, {2, 4, 6, 8}, {1, 2, 3},
+         set(range(1, 40))]
+
+
+@pytest.mark.parametrize("P,Q", [(1, 2), (2, 3), (1, 4), (4, 5), (3, 6),
+                                 (5, 6), (6, 7), (7, 8)])
+@pytest.mark.parametrize("links", LINKS)
+def test_chained_in_part(P, Q, links):
+    N = P + 1
+    for nz in (1, 2, 3, 9, 34):
+        dm, ng = chained_in_part(P, nz, links)
+        J = O.random_jacobians(5, nz)
+        G, Dw = O.geometry_affine(J, Q)
+        tab, x = O.basis_tables(P, Q), O.uniform(11, ng)
+        for op, code, dtype in (("mass", F.OP_MASS, torch.float64),
+                                ("stiffness", F.OP_STIFFNESS, torch.float32)):
+            ref = O.global_operator(op, N, Q, tab, x, dm, G, Dw)
+
+            def dev(a):
+                return torch.from_numpy(np.ascontiguousarray(a)).to("cuda",
+                                                                    dtype)
+            y = torch.empty(ng, device="cuda", dtype=dtype)
+            F.global_apply(code, dev(tab), dev(x), y,
+                           torch.from_numpy(dm).cuda(), nz, P, Q, G=dev(G),
+                           detJw=dev(Dw))
+            torch.cuda.synchronize()
+            got = y.double().cpu().numpy()
+            err = np.linalg.norm(got - ref) / np.linalg.norm(ref)
+            assert err <= TOL[dtype], (op, P, Q, nz, links, err)
+
+
+def test_no_loss_where_nothing_chains():
+    """FP32 mass P=7 on cells whose local axes are rotated, so that the cells
+    after one another share their a-faces and the dofs run along a: as many
+    atomics as dofs of the cells, but no more than 3 times the time of the
+    numbering that chains (5 times when every cell was written in runs along
+    c; 1.4 when its lanes write it)."""
+    P, Q, n = 7, 8, 20
+    N, C = P + 1, n ** 3
+    dm, ng = numbered("lex", (n, n, n), P)
+    rot = np.ascontiguousarray(
+        dm.reshape(C, N, N, N).transpose(0, 3, 1, 2).ravel())
+    tab = torch.from_numpy(O.basis_tables(P, Q)).to("cuda", torch.float32)
+    D = torch.rand(C * Q ** 3, device="cuda")
+    x = torch.rand(ng, device="cuda")
+    y = torch.empty_like(x)
+    ms = []
+    for m in (dm, rot):
+        m = torch.from_numpy(m).cuda()
+        best = 1e9
+        for _ in range(6):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            for _ in range(10):
+                F.global_apply(F.OP_MASS, tab, x, y, m, C, P, Q, detJw=D)
+            b.record()
+            torch.cuda.synchronize()
+            best = min(best, a.elapsed_time(b))
+        ms.append(best)
+    assert ms[1] <= 3 * ms[0], ms
