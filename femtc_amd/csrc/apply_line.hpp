@@ -334,30 +334,56 @@ struct LineStage
   static constexpr int NCH = (Q + CH - 1) / CH;
 };
 
-// Whether the geometry of a stiffness or K+M cell is staged through LDS:
-// wherever two chunks of two points fit the cell's slices (N >= 14, and
-// N >= 12 at Q = N + 2), up to 4 Q + N = 118 for FP32 K+M.  Measured on 20 M
-// dofs against reading it by the line with the next point in flight: FP64
-// stiffness N=14 1.20x, N=16 1.24x, N=17 1.16x, N=18 1.00x, N=20 1.08x, K+M
-// N=16 1.36x; FP32 stiffness N=14..21 1.17-1.32x; against the deepest
-// prefetch that fits the registers (line_geo_depth) 1.0-1.25x.  FP32 K+M
-// N=24 spills: 0.98x, by the line 1.07x.
+// Whether the geometry of a stiffness or K+M cell can be staged through LDS:
+// two chunks of two points fit the cell's two slices at N = 12 and 13 with Q =
+// 14 and from N = 14 on, and staging gains there: against the deepest prefetch
+// by the line (line_geo_depth) at 4e7 values FP64 stiffness 1.04-1.26x, K+M
+// 1.01-1.26x, FP32 1.01-1.28x.  Left by the line, as it measured 0.91-1.02x:
+// FP64 stiffness at Q = 17..19 (but for (15, 17), (17, 17) and (17, 18)), FP32
+// stiffness at Q = 24 (N = 22..24) and FP32 K+M beyond 4 Q + N = 112.
 template <typename T, int OP, int N, int Q>
 constexpr bool line_staged()
 {
-  return (OP == OP_STIFF ||
-          (OP == OP_KPM && (sizeof(T) == 8 || 4 * Q + N <= 118))) &&
-         2 * LineStage<N, Q, 2>::BUF * sizeof(Piece<T>) <=
-             line_cell_lds<T, N, Q>();
+  constexpr bool f64 = sizeof(T) == 8;
+  if (OP != OP_STIFF && OP != OP_KPM)
+    return false;
+  if (line_nbuf<T, N, Q>() < 2 || 2 * LineStage<N, Q, 2>::BUF * sizeof(Piece<T>) >
+                                      line_cell_lds<T, N, Q>())
+    return false;
+  if (OP == OP_KPM)
+    return f64 || 4 * Q + N <= 112;
+  if (!f64)
+    return Q != 24;
+  return Q < 17 || Q > 19 || N == 15 || (N == 17 && Q < 19);
+}
+
+// Workgroups (cells, or pairs of them) per CU, in quarters, from which the
+// staged form runs; fewer run by the line (0: always staged).  Staging pays
+// its barriers by streaming one cell's geometry while another cell of the CU
+// contracts.  Two cells of a workgroup do so only half a cell apart, and from
+// three pairs per CU on that makes up for the half cell at either end: FP32
+// K+M (17, 19) in step / by the line / half apart, 508 pairs 177 / 127 / 125
+// us, 1017 pairs 341 / 287 / 242; FP32 stiffness (18, 18) at 428 pairs 96 / 94
+// / 103.  FP32 cells alone on a CU wait for every chunk: stiffness (23, 23), 16
+// cells, 59 us staged, 54 by the line, 82 cells 64 / 64; K+M (22, 22), 18 cells,
+// 45 / 43, 93 cells 52 / 55.  FP64 cells gain from the smallest counts on (48
+// cells at (16, 16): K+M 1.12x, stiffness 1.08x).
+template <typename T, int OP, int N, int Q>
+constexpr int line_staged_from()
+{
+  return line_cpb<T, OP, N, Q>() == 2 ? 12
+         : sizeof(T) == 8             ? 0
+         : OP == OP_KPM               ? 1
+                                      : 2;
 }
 
 // Barriers the second cell of a staged two-cell workgroup stays behind the
 // first: half of a cell's barriers (10 transposes, one per chunk, two around
 // them), so that one cell streams its geometry while the other contracts.
-template <typename T, int OP, int N, int Q>
+template <typename T, int OP, int N, int Q, bool STAGED>
 constexpr int line_skew()
 {
-  return line_cpb<T, OP, N, Q>() == 2 && line_staged<T, OP, N, Q>()
+  return STAGED && line_cpb<T, OP, N, Q>() == 2
              ? (12 + LineStage<N, Q, 2>::NCH) / 2
              : 0;
 }
@@ -367,7 +393,7 @@ constexpr int line_skew()
 // 5; affine cells compute theirs).  Against one point, 20 M dofs: FP64
 // stiffness N=10 1.12x, N=13 1.05x, FP32 N=10 1.29x, N=13 1.26x, FP64 mass
 // N=10 1.05x, N=17 1.12x.  One point more than fits spills: FP64 K+M N=12,
-// Q=13 at two points 0.95x.
+// Q=13 at two points 0.95x, stiffness N=13, Q=15 0.96x.
 template <typename T, int OP, int N, int Q>
 constexpr int line_geo_depth()
 {
@@ -377,9 +403,11 @@ constexpr int line_geo_depth()
   if (B == OP_MASS)
     return 5;
   constexpr int per = (B == OP_STIFF ? 6 : 7) * (int)(sizeof(T) / 4);
-  constexpr int d = (line_budget(line_waves<T, OP, N, Q>()) -
-                     line_vgprs<T, OP, N, Q>() + 4) /
-                    per;
+  constexpr int room = line_budget(line_waves<T, OP, N, Q>()) -
+                       line_vgprs<T, OP, N, Q>();
+  if (sizeof(T) == 8 && B == OP_STIFF && room < 30)
+    return 1;
+  constexpr int d = (room + 4) / per;
   return d < 1 ? 1 : d > 5 ? 5 : d;
 }
 
@@ -574,7 +602,7 @@ line_pointwise_staged(const T* __restrict__ G, const T* __restrict__ detJw,
   lds_barrier(); // the chunks are read; the slices may be rewritten
 }
 
-template <typename T, int OP, int N, int Q>
+template <typename T, int OP, int N, int Q, bool STAGED>
 __global__ void __launch_bounds__((line_threads<T, OP, N, Q>()))
     __attribute__((amdgpu_waves_per_eu(line_waves<T, OP, N, Q>(),
                                        line_waves<T, OP, N, Q>())))
@@ -602,18 +630,15 @@ __global__ void __launch_bounds__((line_threads<T, OP, N, Q>()))
   const T* const phi = tab; // [dof][q]
   const T* const dph = tab + N * Q;
 
-  // The two cells of a staged workgroup run SKEW barriers apart where the
-  // workgroup takes several pairs: the second cell's waves wait at SKEW extra
-  // barriers before their first cell, the first cell's at as many after
-  // their last, so every wave arrives at the same number.  The cells share
-  // no LDS; the waves of one cell stay in step.
-  constexpr int SKEW = line_skew<T, OP, N, Q>();
-  const bool skewed = C > (int64_t)gridDim.x * CPB;
+  // The two cells of a staged workgroup run SKEW barriers apart: the second
+  // cell's waves wait at SKEW extra barriers before their first cell, the
+  // first cell's at as many after their last, so every wave arrives at the
+  // same number.  The cells share no LDS; the waves of one cell stay in step.
+  constexpr int SKEW = line_skew<T, OP, N, Q, STAGED>();
   auto skew = [&](bool second) {
     if constexpr (SKEW > 0)
     {
-      if (skewed &&
-          (__builtin_amdgcn_readfirstlane(threadIdx.x) >= S::TH) == second)
+      if ((__builtin_amdgcn_readfirstlane(threadIdx.x) >= S::TH) == second)
       {
 #pragma unroll 1
         for (int i = 0; i < SKEW; ++i)
@@ -831,7 +856,7 @@ __global__ void __launch_bounds__((line_threads<T, OP, N, Q>()))
       __syncthreads();
       r_ab_c(4, l);
       line_fwd<T, N, Q>(phi, l, DA);
-      if constexpr (line_staged<T, OP, N, Q>())
+      if constexpr (STAGED)
         line_pointwise_staged<T, OP, N, Q>(G, detJw, cell, t, tab_, slice0, DA,
                                            DB, DC, U);
       else
@@ -924,36 +949,41 @@ __global__ void __launch_bounds__((line_threads<T, OP, N, Q>()))
   skew(false);
 }
 
+template <typename T, int OP, int N, int Q, bool STAGED>
+int line_launch_form(const ApplyReq& r, int64_t grid)
+{
+  hipLaunchKernelGGL((line_cells<T, OP, N, Q, STAGED>), dim3((unsigned)grid),
+                     dim3(line_threads<T, OP, N, Q>()),
+                     (line_lds_bytes<T, OP, N, Q>()), r.stream, (const T*)r.tab,
+                     (const T*)r.x, (T*)r.y, (const T*)r.G, (const T*)r.detJw,
+                     r.gather ? r.dofmap : nullptr, r.num_cells);
+  return hipGetLastError() == hipSuccess ? FEMTC_OK : FEMTC_ERR_HIP;
+}
+
 // Launch for one (N, Q): the op and dtype from the request.
 template <typename T, int OP, int N, int Q>
 int line_launch_op(const ApplyReq& r, int max_lds)
 {
-  constexpr size_t bytes = line_lds_bytes<T, OP, N, Q>();
-  if (bytes > (size_t)max_lds)
+  if (line_lds_bytes<T, OP, N, Q>() > (size_t)max_lds)
     return FEMTC_ERR_INVALID_ARGUMENT;
   constexpr int CPB = line_cpb<T, OP, N, Q>();
-  int64_t grid64 = std::min<int64_t>((r.num_cells + CPB - 1) / CPB, 16384);
-  if constexpr (line_skew<T, OP, N, Q>() > 0)
+  const int64_t groups = (r.num_cells + CPB - 1) / CPB;
+  const int64_t grid = std::min<int64_t>(groups, 16384);
+  if constexpr (line_staged<T, OP, N, Q>())
   {
-    // One workgroup of two staged cells is resident on a CU (10 waves or
-    // more, over 96 VGPRs).  From four pairs per CU on, one workgroup per CU
-    // takes all of them with its cells a half apart; fewer pairs do not make
-    // up for the half cell at either end.  20 M dofs, in step / a half
-    // apart: FP64 stiffness N=17 519 / 448 us; FP32 stiffness N=17 374 / 351,
-    // K+M 469 / 390.
+    constexpr int FROM = line_staged_from<T, OP, N, Q>();
+    if constexpr (FROM == 0)
+      return line_launch_form<T, OP, N, Q, true>(r, grid);
     int dev = 0, cus = 0;
     if (hipGetDevice(&dev) == hipSuccess &&
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount,
                               dev) == hipSuccess &&
-        cus > 0 && grid64 >= 4 * (int64_t)cus)
-      grid64 = cus;
+        cus > 0 && 4 * groups >= (int64_t)FROM * cus)
+      // one workgroup of two staged cells is resident on a CU (10 waves or
+      // more, over 96 VGPRs) and takes all of the CU's pairs
+      return line_launch_form<T, OP, N, Q, true>(r, CPB == 2 ? cus : grid);
   }
-  hipLaunchKernelGGL((line_cells<T, OP, N, Q>), dim3((unsigned)grid64),
-                     dim3(line_threads<T, OP, N, Q>()), bytes, r.stream,
-                     (const T*)r.tab, (const T*)r.x, (T*)r.y, (const T*)r.G,
-                     (const T*)r.detJw, r.gather ? r.dofmap : nullptr,
-                     r.num_cells);
-  return hipGetLastError() == hipSuccess ? FEMTC_OK : FEMTC_ERR_HIP;
+  return line_launch_form<T, OP, N, Q, false>(r, grid);
 }
 
 template <typename T, int OP, int N, int Q>

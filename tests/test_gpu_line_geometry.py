@@ -77,3 +77,53 @@ def test_line_geometry_vs_general(op, dt, P, Q, ncell, apart):
     # norm over all of them
     d = (a - b).view(ncell, nl).norm(dim=1) / b.view(ncell, nl).norm(dim=1)
     assert d.max().item() <= TOL[dt], (op, P, Q, int(d.argmax()))
+
+
+# (P, Q, cells per CU, cells more): either side of the counts from which a
+# shape is staged -- 3 pairs per CU for two cells of a workgroup, half and a
+# quarter of a cell per CU for FP32 stiffness and K+M of one -- and the smallest
+# staged shapes with their neighbours by the line
+EDGES = [
+    (16, 17, 6, -2), (16, 17, 6, -1), (16, 17, 6, 1), (14, 17, 6, 1),
+    (17, 20, 6, -3), (17, 20, 6, 0), (21, 22, 0.5, -1), (21, 22, 0.5, 0),
+    (22, 23, 0.25, -1), (22, 23, 0.25, 0), (11, 14, 0.5, -1),
+    (11, 14, 0.5, 1), (11, 14, 0, 1), (12, 14, 0, 37), (12, 15, 0, 37),
+    (15, 17, 0, 1029), (15, 18, 0, 37), (17, 18, 0, 37), (21, 24, 0, 13),
+]
+
+
+@pytest.mark.parametrize("P,Q,per_cu,more", EDGES)
+@pytest.mark.parametrize("dt", [torch.float64, torch.float32],
+                         ids=["f64", "f32"])
+@pytest.mark.parametrize("op", ["stiffness", "kpm"])
+def test_line_geometry_edges(op, dt, P, Q, per_cu, more):
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    test_line_geometry_vs_general(op, dt, P, Q, int(per_cu * cus) + more,
+                                  False)
+
+
+def test_few_pairs_per_cu():
+    """FP32 K+M at P=16, Q=19 (two cells of 6 waves each) takes about as long
+    per cell with 2 pairs of cells per CU as with 8: 1.2 times, and 1.5 times
+    when the pairs were staged in step."""
+    P, Q = 16, 19
+    N = P + 1
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    tab = torch.from_numpy(O.basis_tables(P, Q)).to("cuda", torch.float32)
+    per_cell = []
+    for C in (4 * cus - 8, 16 * cus):
+        U = torch.rand(C * N ** 3, device="cuda")
+        W = torch.empty_like(U)
+        G = torch.rand(C * Q ** 3 * 6, device="cuda")
+        D = torch.rand(C * Q ** 3, device="cuda")
+        best = 1e9
+        for _ in range(6):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            for _ in range(5):
+                F.kpm_apply(tab, U, W, G, D, C, P, Q)
+            b.record()
+            torch.cuda.synchronize()
+            best = min(best, a.elapsed_time(b))
+        per_cell.append(best / C)
+    assert per_cell[0] <= 1.35 * per_cell[1], per_cell
