@@ -668,8 +668,8 @@ struct femtc_solver
   double* dinv64 = nullptr;
   double* r64 = nullptr;
   double* Au64 = nullptr;
-  double* part = nullptr;
-  double* epart2 = nullptr; // block partials of the operator's energies
+  double* part = nullptr; // block partials: two of the update, then the
+                          // operator's energies (NBLK each)
   int nblk = 1;             // blocks of the vector kernels
   int npart = 1;            // partials the last update launch writes
   double* dscal = nullptr; // device scalar for norms
@@ -764,7 +764,6 @@ void destroy(femtc_solver* S)
   dev_free(S->r64);
   dev_free(S->Au64);
   dev_free(S->part);
-  dev_free(S->epart2);
   dev_free(S->dscal);
   dev_free(S->dbad);
   dev_free(S->st);
@@ -854,6 +853,16 @@ ApplyReq inner_req(const femtc_solver* S, int dtype, const void* x, void* y)
   return a;
 }
 
+// Whether the problem's options leave the z-run scatter open (which also
+// needs the structured numbering).
+bool zrun_allowed(const femtc_solver* S)
+{
+  return S->Q <= 8 && S->prob.grid[0] > 0 && S->prob.grid[1] > 0 &&
+         S->prob.grid[2] > 0 &&
+         (S->prob.scatter == FEMTC_SCATTER_AUTO ||
+          S->prob.scatter == FEMTC_SCATTER_ZRUN);
+}
+
 // Energy partials of the inner operator's z-run launch in precision dtype:
 // one per wave of each z-segment's workgroup.
 int zrun_partials(const femtc_solver* S, int dtype, int64_t* npart)
@@ -921,17 +930,18 @@ LatticeGrid lattice_grid(const femtc_solver* S)
 
 // The vector update of a CG iteration in precision V after the operator:
 // k_update on the atomically scattered Ap, or k_assemble_update on the
-// assembled scatter's cell values.
+// assembled scatter's cell values.  p.Ap is the sum of the nepart energies.
 template <typename V>
-int launch_update(femtc_solver* S, hipStream_t s)
+int launch_update(femtc_solver* S, const double* epart, int64_t nepart,
+                  hipStream_t s)
 {
-  const bool direct = S->nepart <= EPART_DIRECT;
-  const double* energy = direct ? S->epart : S->epart2;
+  const bool direct = nepart <= EPART_DIRECT;
+  const double* energy = direct ? epart : S->part + 2 * NBLK;
   const int nenergy =
-      direct ? (int)S->nepart : std::min(S->nblk, vec_blocks(S->nepart));
+      direct ? (int)nepart : std::min(S->nblk, vec_blocks(nepart));
   if (!direct)
     hipLaunchKernelGGL(k_energy_partials, dim3(nenergy), dim3(RB), 0, s,
-                       (const double*)S->epart, S->nepart, S->epart2,
+                       epart, nepart, S->part + 2 * NBLK,
                        (const PcgState*)S->st);
   if (S->inner_assembled)
   {
@@ -973,19 +983,17 @@ int launch_update(femtc_solver* S, hipStream_t s)
   return hip_status(hipGetLastError());
 }
 
-// Mean time in ms of reps operator-and-update steps (after one warm-up).
+// Mean time in ms of reps operator-and-update steps (after one warm-up), the
+// operator with its energies: without them a direct one would run on another
+// kernel than in the solve.  The update takes D^-1 in their place, whose sum
+// is positive: r.z and p are zero, so alpha is.
 template <typename V>
-int time_step(femtc_solver* S, int reps, float* ms)
+int time_step(femtc_solver* S, hipEvent_t e0, hipEvent_t e1, int reps,
+              float* ms)
 {
-  hipEvent_t e0, e1;
-  if (hipEventCreate(&e0) != hipSuccess)
-    return fail(FEMTC_ERR_HIP, "event creation failed");
-  if (hipEventCreate(&e1) != hipSuccess)
-  {
-    (void)hipEventDestroy(e0);
-    return fail(FEMTC_ERR_HIP, "event creation failed");
-  }
-  const ApplyReq a = inner_req(S, dtype_of<V>(), S->p, S->Ap);
+  ApplyReq a = inner_req(S, dtype_of<V>(), S->p, S->Ap);
+  a.skip = &S->st->done;
+  a.energy = S->epart;
   int st = FEMTC_OK;
   for (int i = 0; i <= reps && st == FEMTC_OK; ++i)
   {
@@ -994,14 +1002,13 @@ int time_step(femtc_solver* S, int reps, float* ms)
     if (st == FEMTC_OK)
       st = run_inner(S, a);
     if (st == FEMTC_OK)
-      st = launch_update<V>(S, S->stream);
+      st = launch_update<V>(S, S->dinv64, std::min(S->nepart, S->n),
+                            S->stream);
   }
   if (st == FEMTC_OK && (hipEventRecord(e1, S->stream) != hipSuccess ||
                          hipEventSynchronize(e1) != hipSuccess ||
                          hipEventElapsedTime(ms, e0, e1) != hipSuccess))
     st = FEMTC_ERR_HIP;
-  (void)hipEventDestroy(e0);
-  (void)hipEventDestroy(e1);
   if (st == FEMTC_ERR_HIP)
     return fail(st, std::string("solver scatter timing: ") +
                         hipGetErrorString(hipGetLastError()));
@@ -1019,6 +1026,27 @@ int64_t energy_partials(int64_t C, int Q, bool assembled, int dtype)
                 : direct_cells(Q);
   const int64_t waves = (cpg * Qq + 63) / 64;
   return (C + cpg - 1) / cpg * waves;
+}
+
+// Selects the inner operator's scatter (0 direct, 1 assembled, 2 z-run) and
+// contraction form, and the number of energy partials its launch writes.
+int set_variant(femtc_solver* S, int scatter, bool even_odd)
+{
+  S->inner_assembled = scatter == 1;
+  S->inner_zrun = scatter == 2;
+  S->even_odd = even_odd;
+  S->nepart = energy_partials(S->prob.num_cells, S->Q, S->inner_assembled,
+                              S->inner_dtype);
+  if (S->inner_zrun)
+  {
+    const int st = zrun_partials(S, S->inner_dtype, &S->nepart);
+    if (st != FEMTC_OK)
+      return st;
+  }
+  if (S->nepart > S->nepart_cap)
+    return fail(FEMTC_ERR_INVALID_ARGUMENT,
+                "solver: more energy partials than were allocated");
+  return FEMTC_OK;
 }
 
 // Scatter and contraction form of the operators.  The scatters allowed by
@@ -1052,9 +1080,7 @@ int choose_variant(femtc_solver* S, int structured)
   const bool have_eo = S->eo64 && S->eo_in;
   bool try_asm = structured && (mode == FEMTC_SCATTER_AUTO ||
                                 mode == FEMTC_SCATTER_ASSEMBLED);
-  const bool try_zrun = structured && S->Q <= 8 &&
-                        (mode == FEMTC_SCATTER_AUTO ||
-                         mode == FEMTC_SCATTER_ZRUN);
+  const bool try_zrun = structured && zrun_allowed(S);
   if (try_asm)
   {
     const size_t es = S->inner_dtype == FEMTC_F64 ? 8 : 4;
@@ -1101,50 +1127,36 @@ int choose_variant(femtc_solver* S, int structured)
       if (st == FEMTC_OK)
         st = fill_zero(v, S->n, dt, s);
     PcgState h{};
-    // the update's alpha = r.z / p.Ap must come out as 0: r.z is, and one
-    // positive energy keeps p.Ap from being
-    if (st == FEMTC_OK)
-      st = fill_zero(S->epart, S->nepart_cap, FEMTC_F64, s);
     if (st == FEMTC_OK &&
-        (hipMemcpyAsync(S->epart, S->dinv64, 8, hipMemcpyDeviceToDevice, s) !=
-             hipSuccess ||
-         hipMemcpyAsync(S->st, &h, sizeof(h), hipMemcpyHostToDevice, s) !=
+        (hipMemcpyAsync(S->st, &h, sizeof(h), hipMemcpyHostToDevice, s) !=
              hipSuccess ||
          hipStreamSynchronize(s) != hipSuccess))
       st = fail(FEMTC_ERR_HIP, "solver: state upload failed");
+    hipEvent_t e0 = nullptr, e1 = nullptr;
+    if (st == FEMTC_OK && (hipEventCreate(&e0) != hipSuccess ||
+                           hipEventCreate(&e1) != hipSuccess))
+      st = fail(FEMTC_ERR_HIP, "event creation failed");
     float tbest = 0.f;
     for (size_t c = 0; c < cand.size() && st == FEMTC_OK; ++c)
     {
-      S->inner_assembled = cand[c].first == 1;
-      S->inner_zrun = cand[c].first == 2;
-      S->even_odd = cand[c].second;
+      if ((st = set_variant(S, cand[c].first, cand[c].second)) != FEMTC_OK)
+        break;
       float t = 0.f;
-      st = dt == FEMTC_F64 ? time_step<double>(S, 3, &t)
-                           : time_step<float>(S, 3, &t);
+      st = dt == FEMTC_F64 ? time_step<double>(S, e0, e1, 3, &t)
+                           : time_step<float>(S, e0, e1, 3, &t);
       if (c == 0 || t < tbest)
       {
         tbest = t;
         best = c;
       }
     }
+    if (e0)
+      (void)hipEventDestroy(e0);
+    if (e1)
+      (void)hipEventDestroy(e1);
   }
-  S->inner_assembled = cand[best].first == 1;
-  S->inner_zrun = cand[best].first == 2;
-  S->even_odd = cand[best].second;
-  S->nepart = energy_partials(S->prob.num_cells, S->Q, S->inner_assembled,
-                              S->inner_dtype);
-  if (S->inner_zrun && st == FEMTC_OK)
-    st = zrun_partials(S, S->inner_dtype, &S->nepart);
-  if (st == FEMTC_OK && S->nepart > S->nepart_cap)
-  {
-    // the z-run launch has a wave per segment slot: more partials
-    dev_free(S->epart);
-    S->bytes -= 8 * (size_t)S->nepart_cap;
-    S->epart = nullptr;
-    S->nepart_cap = 0;
-    if ((st = dev_alloc(S, (void**)&S->epart, 8 * S->nepart)) == FEMTC_OK)
-      S->nepart_cap = S->nepart;
-  }
+  if (st == FEMTC_OK)
+    st = set_variant(S, cand[best].first, cand[best].second);
   if (!S->inner_assembled && S->lattice)
   {
     dev_free(S->lattice);
@@ -1205,7 +1217,7 @@ int enqueue_batch(femtc_solver* S, hipStream_t s)
     int st = run_inner(S, a);
     if (st != FEMTC_OK)
       return st;
-    if ((st = launch_update<V>(S, s)) != FEMTC_OK)
+    if ((st = launch_update<V>(S, S->epart, S->nepart, s)) != FEMTC_OK)
       return st;
     hipLaunchKernelGGL(k_pupdate<V>, dim3(S->nblk), dim3(RB), 0, s, (V*)S->p,
                        (V*)S->e, (const V*)S->r,
@@ -1439,22 +1451,13 @@ int femtc_solver_create(femtc_solver** out, const femtc_problem* prob,
         (st = dev_alloc(S, (void**)&S->dinv64, 8 * n)) ||
         (st = dev_alloc(S, (void**)&S->r64, 8 * n)) ||
         (st = dev_alloc(S, (void**)&S->Au64, 8 * n)) ||
-        (st = dev_alloc(S, (void**)&S->part, 8 * 2 * NBLK)) ||
-        (st = dev_alloc(S, (void**)&S->epart2, 8 * NBLK)) ||
+        (st = dev_alloc(S, (void**)&S->part, 8 * 3 * NBLK)) ||
         (st = dev_alloc(S, (void**)&S->dscal, 8)) ||
         (st = dev_alloc(S, (void**)&S->dbad, sizeof(int))) ||
         (st = dev_alloc(S, (void**)&S->st, sizeof(PcgState))) ||
         (st = dev_alloc(S, &S->rhs, vs * n)) || (st = dev_alloc(S, &S->e, vs * n)) ||
         (st = dev_alloc(S, &S->p, vs * n)) || (st = dev_alloc(S, &S->Ap, vs * n)))
       break;
-    // one energy partial per wave of the operator launch, whose cell
-    // groups depend on the scatter (set again once it is chosen)
-    S->nepart = bf ? C
-                   : std::max(energy_partials(C, S->Q, false, inner_dtype),
-                              energy_partials(C, S->Q, true, inner_dtype));
-    if ((st = dev_alloc(S, (void**)&S->epart, 8 * S->nepart)))
-      break;
-    S->nepart_cap = S->nepart;
     if (hipHostMalloc((void**)&S->hst, sizeof(PcgState)) != hipSuccess ||
         hipHostMalloc((void**)&S->hscal, sizeof(double)) != hipSuccess)
     {
@@ -1467,6 +1470,20 @@ int femtc_solver_create(femtc_solver** out, const femtc_problem* prob,
     S->outer_affine =
         aff && ((prob->op != FEMTC_OP_MASS && !prob->G) ||
                 (prob->op != FEMTC_OP_STIFFNESS && !prob->detJw));
+    // one energy partial per wave of the operator launch, whose cell groups
+    // depend on the scatter: room for any that choose_variant may time
+    S->nepart = bf ? C
+                   : std::max(energy_partials(C, S->Q, false, inner_dtype),
+                              energy_partials(C, S->Q, true, inner_dtype));
+    if (!bf && zrun_allowed(S))
+    {
+      int64_t z = 0;
+      if (zrun_partials(S, inner_dtype, &z) == FEMTC_OK)
+        S->nepart = std::max(S->nepart, z);
+    }
+    if ((st = dev_alloc(S, (void**)&S->epart, 8 * S->nepart)))
+      break;
+    S->nepart_cap = S->nepart;
     const int64_t ntab = 2 * (int64_t)S->N * S->Q;
     if (aff)
     {

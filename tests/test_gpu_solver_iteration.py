@@ -73,3 +73,37 @@ def test_breakdown(inner, scatter):
         for _ in range(2):
             info = S.solve(f, u, rtol=1e-10, maxit=500, check=False)
             assert info["status"] == F._lib.ERR_BREAKDOWN, info
+
+
+def operator_kernels(call):
+    """Names of the operator kernels that call() launches."""
+    from torch.profiler import ProfilerActivity, profile
+
+    torch.cuda.synchronize()
+    with profile(activities=[ProfilerActivity.CUDA]) as prof:
+        call()
+        torch.cuda.synchronize()
+    return {e.key for e in prof.key_averages()
+            if "apply_cells<" in e.key or "chain_cells<" in e.key}
+
+
+@pytest.mark.parametrize("inner", [F.F64, F.F32])
+@pytest.mark.parametrize("structured", [True, False])
+def test_timed_operators_are_the_solves(inner, structured):
+    """The scatters and forms tried at creation are timed on the kernels that
+    a CG iteration launches (which write the energies of p.Ap): not on the
+    chain kernel, which has none, and the chosen one among them."""
+    p = problem((6, 6, 6), 3)
+    if not structured:
+        p["dims"] = None
+    made = []
+    tried = operator_kernels(
+        lambda: made.append(solver(p, inner, F.SCATTER_AUTO)))
+    assert tried and not any("chain_cells" in k for k in tried), tried
+    f = torch.from_numpy(O.uniform(7, p["ng"])).cuda()
+    u = torch.empty_like(f)
+    with made[0] as S:
+        S.set_batch(4, False)
+        run = operator_kernels(lambda: S.solve(f, u, rtol=1e-10))
+    assert {k for k in run if "apply_cells" in k} <= tried, (run, tried)
+    assert any("apply_cells" in k for k in run)
