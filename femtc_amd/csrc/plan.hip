@@ -358,9 +358,12 @@ int plan_request(const femtc_plan* pl, int op, int dtype, int nq,
   r.Q = nq;
   r.gather = 1;
   r.tab = tables;
-  // the even-odd instances cover the direct and assembled scatters; where
-  // the chain kernel takes the direct one, its merged faces are worth more
-  // than half-size products
+  // The even-odd instances cover the direct and assembled scatters; where
+  // the chain kernel takes the direct one, it runs there in general form.
+  // Time of the even-odd atomic scatter over the chain kernel's, every such
+  // shape at nq = degree + 1, 3e6 dofs: lexicographic 1.18-3.4, reader order
+  // 1.5-3.5, cells shuffled, along another axis or with rotated local axes
+  // 0.97-1.13, plates of one cell 0.98-1.35.
   const bool direct_eo = s.x == 0 && !chain_pays(op, dtype == FEMTC_F64, r.N, nq);
   r.eo_tab = (direct_eo || s.x == -1) && nq == r.N ? eo : nullptr;
   r.x = x;

@@ -40,7 +40,9 @@ class Plan:
 
     def set_tables(self, tables, nq: int, stream=None) -> bool:
         """Register a copy of `tables` (its dtype) for applies passing
-        tables=None; True when they contract in even-odd form."""
+        tables=None; True when an even-odd set was made of it, in whose form
+        the assembled scatter, and the direct one where it runs on the atomic
+        kernel, then contract."""
         eo = C.c_int32()
         _lib.check(_lib.lib().femtc_plan_set_tables(
             self._h, _dtype_code(tables), nq, _ptr(tables), _stream(stream),

@@ -350,7 +350,7 @@ int femtc_plan_create(femtc_plan** plan, int nx, int ny, int nz, int degree,
                       const int32_t* dofmap, int64_t ndofs, void* stream);
 int femtc_plan_destroy(femtc_plan* plan);
 /* Block shape (cells per axis) for one (nq, dtype, op); 0,0,0 selects the
- * direct atomic scatter, -1,-1,-1 the assembled scatter, -2,-2,-2 the
+ * direct scatter of femtc_global_apply, -1,-1,-1 the assembled scatter, -2,-2,-2 the
  * structured direct scatter (the atomic scatter with the gather and scatter
  * indices in closed form: the dofmap is not read) and -3,-3,-3 the
  * structured z-run scatter (closed-form indices; each workgroup sums a run
@@ -376,10 +376,13 @@ int femtc_plan_apply(const femtc_plan* plan, int op, int dtype, int nq,
  * nq = degree + 1 and the tables are those of a symmetric node set and
  * rule (phi symmetric and dphi antisymmetric under b -> N-1-b,
  * q -> nq-1-q, to 64 rounding units, as femtc_basis_tables makes them),
- * those applies contract each line in even-odd form (half-size products;
- * results equal to rounding) on the direct and assembled scatters;
- * *even_odd (may be NULL) reports whether they do.  No counterpart in the
- * reference. */
+ * an even-odd set is kept as well and *even_odd (may be NULL) is 1, else 0.
+ * Those applies contract each line in even-odd form (half-size products;
+ * results equal to rounding) on the assembled scatter and, where the direct
+ * scatter runs on the atomic kernel (FP64 stiffness and K+M at degree 5 and
+ * above, FP64 K+M at degree 2, everything at degree 8), on that; elsewhere the
+ * direct scatter's chain kernel is faster in the general form.  No
+ * counterpart in the reference. */
 int femtc_plan_set_tables(femtc_plan* plan, int dtype, int nq,
                           const void* tables, void* stream, int* even_odd);
 /* Time every candidate block shape (and the direct and, for the structured

@@ -279,7 +279,10 @@ EO_MESHES = [(3, 5, 5, 1, 2), (3, 5, 9, 2, 3), (5, 3, 6, 3, 4), (3, 5, 5, 4, 5),
 def test_plan_even_odd_vs_oracle(op, nx, ny, nz, P, Q):
     # registered symmetric tables: the even-odd contractions on the direct
     # and the assembled scatter, FP64 and FP32, overwrite and accumulate,
-    # against the oracle and against the general form on the same plan
+    # against the oracle and against the general form on the same plan.  The
+    # direct scatter runs the chain kernel's general form with either table
+    # set where that is the faster one (the comparison of the two is then of
+    # the kernel with itself); the solver's tests run its even-odd instances
     C, G, Dw, dm, ng = _box(nx, ny, nz, P, Q, 150 + P)
     tab = O.basis_tables(P, Q)
     x = O.uniform(151, ng)

@@ -407,3 +407,26 @@ def test_solver_even_odd_needs_nq_equal_degree_plus_one():
     with F.PCGSolver(op, dev(tab), dev(dm, torch.int32), C, P, Q, ng,
                      G=dev(G), detJw=dev(Dw)) as S:
         assert S.even_odd() is False
+
+
+@pytest.mark.parametrize("P", range(1, 9))
+@pytest.mark.parametrize("op,name", [(F.OP_MASS, "mass"), (F.OP_KPM, "kpm"),
+                                     (F.OP_STIFFNESS, "stiffness")])
+@pytest.mark.parametrize("inner", [F.F64, F.F32])
+def test_direct_even_odd_instances(inner, op, name, P):
+    """The even-odd instances of the atomic scatter, every degree, type and
+    operator (a plan's direct scatter runs the general form on the chain
+    kernel at most of them): f = A x, solved to 1e-8 and checked by the
+    oracle's operator (K is singular; its f is in its range)."""
+    nx, ny, nz = (3, 3, 2) if P < 5 else (2, 2, 2)
+    C, G, Dw, dm, ng, tab, _ = _problem(op, nx, ny, nz, P, P + 1, 230 + P)
+    x = O.uniform(231, ng)
+    f = O.global_operator(name, P + 1, P + 1, tab, x, dm, G, Dw)
+    with F.PCGSolver(op, dev(tab), dev(dm, torch.int32), C, P, P + 1, ng,
+                     G=dev(G), detJw=dev(Dw), inner=inner,
+                     scatter=F.SCATTER_DIRECT, even_odd=True) as S:
+        assert S.even_odd() is True and S.scatter() == F.SCATTER_DIRECT
+        u = torch.empty(ng, device="cuda", dtype=torch.float64)
+        S.solve(dev(f), u, rtol=1e-8)
+    r = O.global_operator(name, P + 1, P + 1, tab, host(u), dm, G, Dw)
+    assert rel(r, f) <= 1.05e-8
