@@ -40,7 +40,6 @@ ApplyLauncher chain_launcher_for(int N)
   case 6: return launch_chain_n6;
   case 7: return launch_chain_n7;
   case 8: return launch_chain_n8;
-  case 9: return launch_chain_n9;
   }
   return nullptr;
 }

@@ -52,24 +52,21 @@
 namespace femtc
 {
 
-// Waves of a chain workgroup: 4, as far as their work areas and the box leave
-// a second workgroup room on the CU; 2 where a wave holds 7 or 16 cells and
-// two already make long rows (affine FP64 stiffness P=2, 1.6e7 dofs: 403 ->
-// 371 us; mass P=1: 627 -> 557).
-template <typename T, int Q, int OP>
+// Waves of a chain workgroup: 4; 2 where a wave holds 7 or 16 cells and two
+// already make long rows (affine FP64 stiffness P=2, 1.6e7 dofs: 403 -> 371
+// us; mass P=1: 627 -> 557).
+template <int Q>
 constexpr int chain_waves()
 {
-  if (Q <= 3)
-    return 2;
-  return sizeof(T) == 8 && Q == 8 && OP != OP_MASS && OP != OP_MASS_AFF ? 3 : 4;
+  return Q <= 3 ? 2 : 4;
 }
 
 template <typename T, int N, int Q, int OP>
 struct ChainShape
 {
-  using Ch = CellChain<T, N, Q, OP, false>;
+  using Ch = CellChain<T, N, Q, OP>;
   static constexpr int P = N - 1;
-  static constexpr int BT = 64 * chain_waves<T, Q, OP>();
+  static constexpr int BT = 64 * chain_waves<Q>();
   static constexpr bool PACK = Q == 6;         // cells straddle waves
   static constexpr int GT = PACK ? BT : 64;    // threads of a cell group
   static constexpr int NG = BT / GT;           // groups
@@ -102,7 +99,7 @@ struct ChainShape
 };
 
 template <typename T, int N, int Q, int OP>
-__global__ void __launch_bounds__((64 * chain_waves<T, Q, OP>()))
+__global__ void __launch_bounds__((64 * chain_waves<Q>()))
     chain_cells(const T* __restrict__ tab, const T* __restrict__ x,
                 T* __restrict__ y, const T* __restrict__ G,
                 const T* __restrict__ detJw, const int32_t* __restrict__ dofmap,

@@ -117,6 +117,14 @@ constexpr int group_threads()
   return ((cells_per_group<T, Q, BW>() * Q * Q + 63) / 64) * 64;
 }
 
+// Atomic add into LDS (ds_add_f64 / ds_add_f32): lanes of one instruction
+// that hit the same address all count.
+template <typename T>
+__device__ inline void lds_add(T* p, T v)
+{
+  __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
 // Row d of a [rows][LEN] table, loaded at this point of the program: the
 // offset goes through an empty asm so the compiler cannot hoist the (scalar)
 // loads of every row to the top of the kernel.  It is an unsigned byte
@@ -181,6 +189,21 @@ __device__ inline void load_row4(const T* __restrict__ tab, int off, T (&row)[LE
   }
 }
 
+// e[k] = v[k] + v[K-1-k], o[k] = v[k] - v[K-1-k], e[K/2] = v[K/2] (odd K)
+template <int K, typename T>
+__device__ inline void eo_split(const T (&v)[K], T (&e)[(K + 1) / 2],
+                                T (&o)[K / 2])
+{
+#pragma unroll
+  for (int k = 0; k < K / 2; ++k)
+  {
+    e[k] = v[k] + v[K - 1 - k];
+    o[k] = v[k] - v[K - 1 - k];
+  }
+  if constexpr (K % 2)
+    e[K / 2] = v[K / 2];
+}
+
 // One table term (term dims of eo_dims(K, M, S), at element offset off):
 // S = +1: ev += A e, od += B o;  S = -1: ev += A o, od += B e.
 // INIT: the first term into ev/od (products instead of sums).
@@ -218,6 +241,21 @@ __device__ inline void eo_term(const T* __restrict__ tab, int off,
     for (int m = 0; m < d.Hm; ++m)
       od[m] = (INIT && k == 0) ? row[m] * in : fma(row[m], in, od[m]);
   }
+}
+
+// out[m] = ev[m] + od[m], out[M-1-m] = ev[m] - od[m], out[M/2] = ev[M/2]
+template <int M, typename T>
+__device__ inline void eo_join(const T (&ev)[(M + 1) / 2], const T (&od)[M / 2],
+                               T (&out)[M])
+{
+#pragma unroll
+  for (int m = 0; m < M / 2; ++m)
+  {
+    out[m] = ev[m] + od[m];
+    out[M - 1 - m] = ev[m] - od[m];
+  }
+  if constexpr (M % 2)
+    out[M / 2] = ev[M / 2];
 }
 
 // Lane-contiguous pieces of the qa-planes [QB0, QB0+QH) of the geometry of
@@ -1446,7 +1484,7 @@ int launch_cells(const ApplyReq& r)
       return launch_cells<T, N, Q, OP, REF, GATHER, EO, SCATTER_LOCAL>(r);
   }
   constexpr int CPB = cells_per_group<T, Q, BW>();
-  constexpr long long XC = xcd_chunk<T, Q, GATHER>();
+  constexpr long long XC = BW == 0 ? xcd_chunk<T, Q, GATHER>() : 1;
   const long long nblk = (r.num_cells + CPB - 1) / CPB;
   if (nblk == 0)
     return FEMTC_OK;

@@ -7,24 +7,20 @@
 // acc[m] += T[k][m] in[k], and the wave-uniform T[k][m] come from vector
 // registers through dpp_fma (dpp_fma.hpp): the table set is loaded once per
 // wave (2 N Q values in 2 N Q / 16 registers: 14 VGPRs for FP64 at N = Q =
-// 7).  Measured against scalar loads of each row as in apply_kernel.hpp
-// (MI355X, us per gathered apply): affine FP64 K+M at P=5, 97,290 cells, 235
-// -> 218; FP64 mass at P=7 on full z-lines, 68,880 cells, 217 -> 205; FP32
+// 7).  Against scalar loads of each row as in apply_kernel.hpp (MI355X, us
+// per gathered apply): affine FP64 K+M at P=5, 97,290 cells, 235 -> 218; FP32
 // mass at P=3, Q=5, 290,177 cells, 113 -> 110.  (In the fused kernels of
-// apply_kernel.hpp, one cell group per workgroup, scalar rows are as fast or
-// faster: FP32 even-odd cell pass 134 against 166.)
+// apply_kernel.hpp scalar rows are as fast or faster: FP32 even-odd cell pass
+// 134 against 166.)
 //
 // Every stage therefore runs in all lanes of the wave.  Lanes outside a
 // stage's role read a line that another lane owns and have their stores
-// masked (the `on` arguments): a masked read would leave their registers to
-// the previous values, which inside a loop over cells then stay live through
-// the whole body (FP64 stiffness at N = Q = 7: 320 VGPRs instead of 160).
+// masked (the `on` arguments).
 #pragma once
 
 #include "cell_common.hpp"
 #include "common.hpp"
 #include "dpp_fma.hpp"
-#include "even_odd.hpp"
 #include "lds_layout.hpp"
 
 namespace femtc
@@ -70,30 +66,8 @@ __device__ __forceinline__ void clear(T (&a)[M])
     a[m] = T(0);
 }
 
-// One even-odd table term (dims of eo_dims(K, M, S), at element offset OFF):
-// S = +1: ev += A e, od += B o;  S = -1: ev += A o, od += B e.
-template <int K, int M, int S, int OFF, int NR, typename T>
-__device__ __forceinline__ void
-eo_term(const T (&t)[NR], const T (&e)[(K + 1) / 2], const T (&o)[K / 2],
-        T (&ev)[(M + 1) / 2], T (&od)[M / 2])
-{
-  constexpr EoDims d = eo_dims(K, M, S);
-  constexpr int OB = OFF + d.rowsA * d.RA;
-  if constexpr (S > 0)
-  {
-    contract<OFF, d.RA, 1>(t, e, ev);
-    contract<OB, d.RB, 1>(t, o, od);
-  }
-  else
-  {
-    contract<OFF, d.RA, 1>(t, o, ev);
-    contract<OB, d.RB, 1>(t, e, od);
-  }
-}
-
-// One cell's stages for operator OP (correct mode) in precision T.  EO: the
-// table registers hold the even-odd table set.
-template <typename T, int N, int Q, int OP, bool EO>
+// One cell's stages for operator OP (correct mode) in precision T.
+template <typename T, int N, int Q, int OP>
 struct CellChain
 {
   static constexpr bool AFF = OP >= OP_MASS_AFF; // geometry per cell
@@ -101,15 +75,12 @@ struct CellChain
   static constexpr bool MASSTERM = (OPB == OP_MASS || OPB == OP_KPM);
   static constexpr bool GRAD = (OPB != OP_MASS);
   static constexpr bool GEO = GRAD && !AFF; // geometry streamed per point
-  // table registers: [phi | dphi] (phi alone for the mass operator), or the
-  // four even-odd terms
-  static constexpr int TABLE = EO     ? eo_offset(N, Q, EO_WEIGHTS)
-                               : GRAD ? 2 * N * Q
-                                      : N * Q;
+  // table registers: [phi | dphi] (phi alone for the mass operator)
+  static constexpr int TABLE = GRAD ? 2 * N * Q : N * Q;
   using Tab = TableRegs<T, TABLE>;
   static constexpr int NR = Tab::NR;
   // the Gauss weights in the table set in memory
-  static constexpr int WOFF = EO ? eo_offset(N, Q, EO_WEIGHTS) : 2 * N * Q;
+  static constexpr int WOFF = 2 * N * Q;
   static constexpr int NX = GRAD ? 2 : 1; // X tensors
   static constexpr int NY = GRAD ? 3 : 1; // Y tensors
   // X[qb][c][a] and Y[a][qb][qc] with bank-conflict-minimising strides
@@ -134,26 +105,13 @@ struct CellChain
     return X > Y ? X : Y;
   }
 
-  // out += phi in (D = 0) or g in (D = 1), dofs to points
+  // out = phi in (D = 0) or g in (D = 1), dofs to points
   template <int D>
   static __device__ __forceinline__ void fwd(const Tab& t, const T (&in)[N],
                                              T (&out)[Q])
   {
-    if constexpr (EO)
-    {
-      T e[(N + 1) / 2], o[N / 2], ev[(Q + 1) / 2], od[Q / 2];
-      eo_split<N>(in, e, o);
-      clear(ev);
-      clear(od);
-      eo_term<N, Q, D ? -1 : 1, eo_offset(N, Q, D ? EO_DPHI_F : EO_PHI_F)>(
-          t.r, e, o, ev, od);
-      eo_join<Q>(ev, od, out);
-    }
-    else
-    {
-      clear(out);
-      contract<D * N * Q, Q, 1>(t.r, in, out);
-    }
+    clear(out);
+    contract<D * N * Q, Q, 1>(t.r, in, out);
   }
 
   // out = sum of phi' in0 (HAS0) and g' in1 (HAS1), points to dofs
@@ -161,31 +119,11 @@ struct CellChain
   static __device__ __forceinline__ void bwd(const Tab& t, const T (&in0)[Q],
                                              const T (&in1)[Q], T (&out)[N])
   {
-    if constexpr (EO)
-    {
-      T e[(Q + 1) / 2], o[Q / 2], ev[(N + 1) / 2], od[N / 2];
-      clear(ev);
-      clear(od);
-      if constexpr (HAS0)
-      {
-        eo_split<Q>(in0, e, o);
-        eo_term<Q, N, 1, eo_offset(N, Q, EO_PHI_B)>(t.r, e, o, ev, od);
-      }
-      if constexpr (HAS1)
-      {
-        eo_split<Q>(in1, e, o);
-        eo_term<Q, N, -1, eo_offset(N, Q, EO_DPHI_B)>(t.r, e, o, ev, od);
-      }
-      eo_join<N>(ev, od, out);
-    }
-    else
-    {
-      clear(out);
-      if constexpr (HAS0)
-        contract<0, 1, Q>(t.r, in0, out);
-      if constexpr (HAS1)
-        contract<N * Q, 1, Q>(t.r, in1, out);
-    }
+    clear(out);
+    if constexpr (HAS0)
+      contract<0, 1, Q>(t.r, in0, out);
+    if constexpr (HAS1)
+      contract<N * Q, 1, Q>(t.r, in1, out);
   }
 
   // F1: contract axis b of the line (a, c) and store it into X.

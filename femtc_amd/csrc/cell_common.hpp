@@ -19,48 +19,10 @@ __device__ inline void atomic_add(double* p, double v)
 }
 __device__ inline void atomic_add(float* p, float v) { unsafeAtomicAdd(p, v); }
 
-// Atomic add into LDS (ds_add_f64 / ds_add_f32): lanes of one instruction
-// that hit the same address all count.
-template <typename T>
-__device__ inline void lds_add(T* p, T v)
-{
-  __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-}
-
 template <typename T>
 __device__ inline T stream_load(const T* p)
 {
   return __builtin_nontemporal_load(p);
-}
-
-// e[k] = v[k] + v[K-1-k], o[k] = v[k] - v[K-1-k], e[K/2] = v[K/2] (odd K)
-template <int K, typename T>
-__device__ inline void eo_split(const T (&v)[K], T (&e)[(K + 1) / 2],
-                                T (&o)[K / 2])
-{
-#pragma unroll
-  for (int k = 0; k < K / 2; ++k)
-  {
-    e[k] = v[k] + v[K - 1 - k];
-    o[k] = v[k] - v[K - 1 - k];
-  }
-  if constexpr (K % 2)
-    e[K / 2] = v[K / 2];
-}
-
-// out[m] = ev[m] + od[m], out[M-1-m] = ev[m] - od[m], out[M/2] = ev[M/2]
-template <int M, typename T>
-__device__ inline void eo_join(const T (&ev)[(M + 1) / 2], const T (&od)[M / 2],
-                               T (&out)[M])
-{
-#pragma unroll
-  for (int m = 0; m < M / 2; ++m)
-  {
-    out[m] = ev[m] + od[m];
-    out[M - 1 - m] = ev[m] - od[m];
-  }
-  if constexpr (M % 2)
-    out[M / 2] = ev[M / 2];
 }
 
 // The geometry block is staged through LDS in two halves of qa-planes:

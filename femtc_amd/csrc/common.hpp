@@ -235,7 +235,6 @@ int launch_chain_n5(const ApplyReq&);
 int launch_chain_n6(const ApplyReq&);
 int launch_chain_n7(const ApplyReq&);
 int launch_chain_n8(const ApplyReq&);
-int launch_chain_n9(const ApplyReq&);
 // N = 10..26 (apply_general.hip); also accepts smaller N
 int launch_apply_general(const ApplyReq&);
 // Line kernels, N = 10..26 (apply_line.hpp); max_lds = the device's LDS

@@ -175,96 +175,6 @@ __device__ __forceinline__ void dpp_fma(const double (&t)[NR], double x,
 }
 
 template <int OFF, int STRIDE, int NR>
-__device__ __forceinline__ void dpp_fma(const double (&t)[NR], double x,
-                                        double (&a)[9])
-{
-  static_assert(OFF + 8 * STRIDE < 16 * NR, "value inside the table");
-  asm("s_nop 1\n\t"
-      "v_fmac_f64_dpp %0, %9, %27 row_newbcast:%10 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f64_dpp %1, %11, %27 row_newbcast:%12 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f64_dpp %2, %13, %27 row_newbcast:%14 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f64_dpp %3, %15, %27 row_newbcast:%16 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f64_dpp %4, %17, %27 row_newbcast:%18 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f64_dpp %5, %19, %27 row_newbcast:%20 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f64_dpp %6, %21, %27 row_newbcast:%22 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f64_dpp %7, %23, %27 row_newbcast:%24 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f64_dpp %8, %25, %27 row_newbcast:%26 row_mask:0xf bank_mask:0xf"
-      : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]), "+v"(a[4]), "+v"(a[5]), "+v"(a[6]), "+v"(a[7]), "+v"(a[8])
-      : "v"(t[(OFF + 0 * STRIDE) / 16]), "n"((OFF + 0 * STRIDE) % 16),
-        "v"(t[(OFF + 1 * STRIDE) / 16]), "n"((OFF + 1 * STRIDE) % 16),
-        "v"(t[(OFF + 2 * STRIDE) / 16]), "n"((OFF + 2 * STRIDE) % 16),
-        "v"(t[(OFF + 3 * STRIDE) / 16]), "n"((OFF + 3 * STRIDE) % 16),
-        "v"(t[(OFF + 4 * STRIDE) / 16]), "n"((OFF + 4 * STRIDE) % 16),
-        "v"(t[(OFF + 5 * STRIDE) / 16]), "n"((OFF + 5 * STRIDE) % 16),
-        "v"(t[(OFF + 6 * STRIDE) / 16]), "n"((OFF + 6 * STRIDE) % 16),
-        "v"(t[(OFF + 7 * STRIDE) / 16]), "n"((OFF + 7 * STRIDE) % 16),
-        "v"(t[(OFF + 8 * STRIDE) / 16]), "n"((OFF + 8 * STRIDE) % 16),
-        "v"(x));
-}
-
-template <int OFF, int STRIDE, int NR>
-__device__ __forceinline__ void dpp_fma(const double (&t)[NR], double x,
-                                        double (&a)[10])
-{
-  static_assert(OFF + 9 * STRIDE < 16 * NR, "value inside the table");
-  asm("s_nop 1\n\t"
-      "v_fmac_f64_dpp %0, %10, %30 row_newbcast:%11 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f64_dpp %1, %12, %30 row_newbcast:%13 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f64_dpp %2, %14, %30 row_newbcast:%15 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f64_dpp %3, %16, %30 row_newbcast:%17 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f64_dpp %4, %18, %30 row_newbcast:%19 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f64_dpp %5, %20, %30 row_newbcast:%21 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f64_dpp %6, %22, %30 row_newbcast:%23 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f64_dpp %7, %24, %30 row_newbcast:%25 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f64_dpp %8, %26, %30 row_newbcast:%27 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f64_dpp %9, %28, %30 row_newbcast:%29 row_mask:0xf bank_mask:0xf"
-      : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]), "+v"(a[4]), "+v"(a[5]), "+v"(a[6]), "+v"(a[7]), "+v"(a[8]), "+v"(a[9])
-      : "v"(t[(OFF + 0 * STRIDE) / 16]), "n"((OFF + 0 * STRIDE) % 16),
-        "v"(t[(OFF + 1 * STRIDE) / 16]), "n"((OFF + 1 * STRIDE) % 16),
-        "v"(t[(OFF + 2 * STRIDE) / 16]), "n"((OFF + 2 * STRIDE) % 16),
-        "v"(t[(OFF + 3 * STRIDE) / 16]), "n"((OFF + 3 * STRIDE) % 16),
-        "v"(t[(OFF + 4 * STRIDE) / 16]), "n"((OFF + 4 * STRIDE) % 16),
-        "v"(t[(OFF + 5 * STRIDE) / 16]), "n"((OFF + 5 * STRIDE) % 16),
-        "v"(t[(OFF + 6 * STRIDE) / 16]), "n"((OFF + 6 * STRIDE) % 16),
-        "v"(t[(OFF + 7 * STRIDE) / 16]), "n"((OFF + 7 * STRIDE) % 16),
-        "v"(t[(OFF + 8 * STRIDE) / 16]), "n"((OFF + 8 * STRIDE) % 16),
-        "v"(t[(OFF + 9 * STRIDE) / 16]), "n"((OFF + 9 * STRIDE) % 16),
-        "v"(x));
-}
-
-template <int OFF, int STRIDE, int NR>
-__device__ __forceinline__ void dpp_fma(const double (&t)[NR], double x,
-                                        double (&a)[11])
-{
-  static_assert(OFF + 10 * STRIDE < 16 * NR, "value inside the table");
-  asm("s_nop 1\n\t"
-      "v_fmac_f64_dpp %0, %11, %33 row_newbcast:%12 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f64_dpp %1, %13, %33 row_newbcast:%14 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f64_dpp %2, %15, %33 row_newbcast:%16 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f64_dpp %3, %17, %33 row_newbcast:%18 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f64_dpp %4, %19, %33 row_newbcast:%20 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f64_dpp %5, %21, %33 row_newbcast:%22 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f64_dpp %6, %23, %33 row_newbcast:%24 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f64_dpp %7, %25, %33 row_newbcast:%26 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f64_dpp %8, %27, %33 row_newbcast:%28 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f64_dpp %9, %29, %33 row_newbcast:%30 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f64_dpp %10, %31, %33 row_newbcast:%32 row_mask:0xf bank_mask:0xf"
-      : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]), "+v"(a[4]), "+v"(a[5]), "+v"(a[6]), "+v"(a[7]), "+v"(a[8]), "+v"(a[9]), "+v"(a[10])
-      : "v"(t[(OFF + 0 * STRIDE) / 16]), "n"((OFF + 0 * STRIDE) % 16),
-        "v"(t[(OFF + 1 * STRIDE) / 16]), "n"((OFF + 1 * STRIDE) % 16),
-        "v"(t[(OFF + 2 * STRIDE) / 16]), "n"((OFF + 2 * STRIDE) % 16),
-        "v"(t[(OFF + 3 * STRIDE) / 16]), "n"((OFF + 3 * STRIDE) % 16),
-        "v"(t[(OFF + 4 * STRIDE) / 16]), "n"((OFF + 4 * STRIDE) % 16),
-        "v"(t[(OFF + 5 * STRIDE) / 16]), "n"((OFF + 5 * STRIDE) % 16),
-        "v"(t[(OFF + 6 * STRIDE) / 16]), "n"((OFF + 6 * STRIDE) % 16),
-        "v"(t[(OFF + 7 * STRIDE) / 16]), "n"((OFF + 7 * STRIDE) % 16),
-        "v"(t[(OFF + 8 * STRIDE) / 16]), "n"((OFF + 8 * STRIDE) % 16),
-        "v"(t[(OFF + 9 * STRIDE) / 16]), "n"((OFF + 9 * STRIDE) % 16),
-        "v"(t[(OFF + 10 * STRIDE) / 16]), "n"((OFF + 10 * STRIDE) % 16),
-        "v"(x));
-}
-
-template <int OFF, int STRIDE, int NR>
 __device__ __forceinline__ void dpp_fma(const float (&t)[NR], float x,
                                         float (&a)[1])
 {
@@ -413,96 +323,6 @@ __device__ __forceinline__ void dpp_fma(const float (&t)[NR], float x,
         "v"(t[(OFF + 5 * STRIDE) / 16]), "n"((OFF + 5 * STRIDE) % 16),
         "v"(t[(OFF + 6 * STRIDE) / 16]), "n"((OFF + 6 * STRIDE) % 16),
         "v"(t[(OFF + 7 * STRIDE) / 16]), "n"((OFF + 7 * STRIDE) % 16),
-        "v"(x));
-}
-
-template <int OFF, int STRIDE, int NR>
-__device__ __forceinline__ void dpp_fma(const float (&t)[NR], float x,
-                                        float (&a)[9])
-{
-  static_assert(OFF + 8 * STRIDE < 16 * NR, "value inside the table");
-  asm("s_nop 1\n\t"
-      "v_fmac_f32_dpp %0, %9, %27 row_newbcast:%10 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f32_dpp %1, %11, %27 row_newbcast:%12 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f32_dpp %2, %13, %27 row_newbcast:%14 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f32_dpp %3, %15, %27 row_newbcast:%16 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f32_dpp %4, %17, %27 row_newbcast:%18 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f32_dpp %5, %19, %27 row_newbcast:%20 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f32_dpp %6, %21, %27 row_newbcast:%22 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f32_dpp %7, %23, %27 row_newbcast:%24 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f32_dpp %8, %25, %27 row_newbcast:%26 row_mask:0xf bank_mask:0xf"
-      : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]), "+v"(a[4]), "+v"(a[5]), "+v"(a[6]), "+v"(a[7]), "+v"(a[8])
-      : "v"(t[(OFF + 0 * STRIDE) / 16]), "n"((OFF + 0 * STRIDE) % 16),
-        "v"(t[(OFF + 1 * STRIDE) / 16]), "n"((OFF + 1 * STRIDE) % 16),
-        "v"(t[(OFF + 2 * STRIDE) / 16]), "n"((OFF + 2 * STRIDE) % 16),
-        "v"(t[(OFF + 3 * STRIDE) / 16]), "n"((OFF + 3 * STRIDE) % 16),
-        "v"(t[(OFF + 4 * STRIDE) / 16]), "n"((OFF + 4 * STRIDE) % 16),
-        "v"(t[(OFF + 5 * STRIDE) / 16]), "n"((OFF + 5 * STRIDE) % 16),
-        "v"(t[(OFF + 6 * STRIDE) / 16]), "n"((OFF + 6 * STRIDE) % 16),
-        "v"(t[(OFF + 7 * STRIDE) / 16]), "n"((OFF + 7 * STRIDE) % 16),
-        "v"(t[(OFF + 8 * STRIDE) / 16]), "n"((OFF + 8 * STRIDE) % 16),
-        "v"(x));
-}
-
-template <int OFF, int STRIDE, int NR>
-__device__ __forceinline__ void dpp_fma(const float (&t)[NR], float x,
-                                        float (&a)[10])
-{
-  static_assert(OFF + 9 * STRIDE < 16 * NR, "value inside the table");
-  asm("s_nop 1\n\t"
-      "v_fmac_f32_dpp %0, %10, %30 row_newbcast:%11 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f32_dpp %1, %12, %30 row_newbcast:%13 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f32_dpp %2, %14, %30 row_newbcast:%15 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f32_dpp %3, %16, %30 row_newbcast:%17 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f32_dpp %4, %18, %30 row_newbcast:%19 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f32_dpp %5, %20, %30 row_newbcast:%21 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f32_dpp %6, %22, %30 row_newbcast:%23 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f32_dpp %7, %24, %30 row_newbcast:%25 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f32_dpp %8, %26, %30 row_newbcast:%27 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f32_dpp %9, %28, %30 row_newbcast:%29 row_mask:0xf bank_mask:0xf"
-      : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]), "+v"(a[4]), "+v"(a[5]), "+v"(a[6]), "+v"(a[7]), "+v"(a[8]), "+v"(a[9])
-      : "v"(t[(OFF + 0 * STRIDE) / 16]), "n"((OFF + 0 * STRIDE) % 16),
-        "v"(t[(OFF + 1 * STRIDE) / 16]), "n"((OFF + 1 * STRIDE) % 16),
-        "v"(t[(OFF + 2 * STRIDE) / 16]), "n"((OFF + 2 * STRIDE) % 16),
-        "v"(t[(OFF + 3 * STRIDE) / 16]), "n"((OFF + 3 * STRIDE) % 16),
-        "v"(t[(OFF + 4 * STRIDE) / 16]), "n"((OFF + 4 * STRIDE) % 16),
-        "v"(t[(OFF + 5 * STRIDE) / 16]), "n"((OFF + 5 * STRIDE) % 16),
-        "v"(t[(OFF + 6 * STRIDE) / 16]), "n"((OFF + 6 * STRIDE) % 16),
-        "v"(t[(OFF + 7 * STRIDE) / 16]), "n"((OFF + 7 * STRIDE) % 16),
-        "v"(t[(OFF + 8 * STRIDE) / 16]), "n"((OFF + 8 * STRIDE) % 16),
-        "v"(t[(OFF + 9 * STRIDE) / 16]), "n"((OFF + 9 * STRIDE) % 16),
-        "v"(x));
-}
-
-template <int OFF, int STRIDE, int NR>
-__device__ __forceinline__ void dpp_fma(const float (&t)[NR], float x,
-                                        float (&a)[11])
-{
-  static_assert(OFF + 10 * STRIDE < 16 * NR, "value inside the table");
-  asm("s_nop 1\n\t"
-      "v_fmac_f32_dpp %0, %11, %33 row_newbcast:%12 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f32_dpp %1, %13, %33 row_newbcast:%14 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f32_dpp %2, %15, %33 row_newbcast:%16 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f32_dpp %3, %17, %33 row_newbcast:%18 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f32_dpp %4, %19, %33 row_newbcast:%20 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f32_dpp %5, %21, %33 row_newbcast:%22 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f32_dpp %6, %23, %33 row_newbcast:%24 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f32_dpp %7, %25, %33 row_newbcast:%26 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f32_dpp %8, %27, %33 row_newbcast:%28 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f32_dpp %9, %29, %33 row_newbcast:%30 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f32_dpp %10, %31, %33 row_newbcast:%32 row_mask:0xf bank_mask:0xf"
-      : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]), "+v"(a[4]), "+v"(a[5]), "+v"(a[6]), "+v"(a[7]), "+v"(a[8]), "+v"(a[9]), "+v"(a[10])
-      : "v"(t[(OFF + 0 * STRIDE) / 16]), "n"((OFF + 0 * STRIDE) % 16),
-        "v"(t[(OFF + 1 * STRIDE) / 16]), "n"((OFF + 1 * STRIDE) % 16),
-        "v"(t[(OFF + 2 * STRIDE) / 16]), "n"((OFF + 2 * STRIDE) % 16),
-        "v"(t[(OFF + 3 * STRIDE) / 16]), "n"((OFF + 3 * STRIDE) % 16),
-        "v"(t[(OFF + 4 * STRIDE) / 16]), "n"((OFF + 4 * STRIDE) % 16),
-        "v"(t[(OFF + 5 * STRIDE) / 16]), "n"((OFF + 5 * STRIDE) % 16),
-        "v"(t[(OFF + 6 * STRIDE) / 16]), "n"((OFF + 6 * STRIDE) % 16),
-        "v"(t[(OFF + 7 * STRIDE) / 16]), "n"((OFF + 7 * STRIDE) % 16),
-        "v"(t[(OFF + 8 * STRIDE) / 16]), "n"((OFF + 8 * STRIDE) % 16),
-        "v"(t[(OFF + 9 * STRIDE) / 16]), "n"((OFF + 9 * STRIDE) % 16),
-        "v"(t[(OFF + 10 * STRIDE) / 16]), "n"((OFF + 10 * STRIDE) % 16),
         "v"(x));
 }
 

@@ -29,7 +29,7 @@ namespace femtc
 {
 """
 
-MAX = 11
+MAX = 8  # lines of at most 8 dofs or points
 
 
 def block(ctype, op, n):
