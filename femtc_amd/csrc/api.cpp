@@ -53,7 +53,7 @@ ApplyLauncher pick_launcher(const ApplyReq& r)
   const bool atomic = r.gather && !r.reference_mode && !r.blocked &&
                       !r.assembled && !r.structured_direct && !r.zrun &&
                       !r.eo_tab && !r.energy;
-  if (atomic && chain_pays(r.op, r.dtype == FEMTC_F64, r.N, r.Q))
+  if (atomic && chain_runs(r.op, r.dtype == FEMTC_F64, r.N, r.Q, r.num_cells))
     return chain_launcher_for(r.N);
   return launcher_for(r.N);
 }

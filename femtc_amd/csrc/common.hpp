@@ -132,6 +132,44 @@ constexpr bool chain_pays(int op, bool f64, int N, int Q)
                 : Q == N && N <= 5 && !(op == OP_KPM && N == 3);
 }
 
+// Cells from which the chain kernel is the faster one.  Its box, two more
+// barriers and 2-4 waves per workgroup make a chain of cells take up to twice
+// as long as the atomic kernel's cells do, and few cells are all resident at
+// once: time of the atomic scatter over the chain's on lexicographic boxes, at
+// (cells) just below and above the line, lowest and highest over the types and
+// operators:
+//   P=1 Q=2  (8000) 0.94-1.07, (11000) 0.98-1.06   Q=3  (16000) 0.91-1.00,
+//       (24000) 0.97-1.05   FP64 Q=4  (5600) 0.99, (8000) 1.05; FP32 1.02-1.12
+//       from the fewest on
+//   P=2  (4000) 0.86-1.04, (8000) 1.01-1.37
+//   P=3  Q=4  (1400) 0.86-0.95, (2000) 0.98-1.10   (4000) 0.94-1.25, (5600)
+//       0.99-1.44
+//   P=4  Q=5  (2800) 0.95-1.10, (4000) 1.03-1.32   (2800) 0.88-1.06, (4000)
+//       0.97-1.26
+//   P=5  Q=6  (1400) 0.93-1.00, (2000) 1.05-1.34   (2800) 0.89-1.14, (4000)
+//       0.95-1.24
+//   P=6, 7  (1000) 0.83-0.88, (1400) 1.03-1.24
+// Numberings in a reader's order cross at fewer cells; where nothing chains,
+// 1e3 to 3e4 cells, 0.84-1.2 (0.76-0.8 for affine FP64 at P=5, Q=6).
+constexpr long long chain_cells_from(bool f64, int N, int Q)
+{
+  switch (N)
+  {
+  case 2: return Q == 2 ? 10240 : Q == 3 ? 24576 : f64 ? 8192 : 0;
+  case 3: return 6144;
+  case 4: return Q == 4 ? 2048 : 5120;
+  case 5: return Q == 5 ? 3072 : 4096;
+  case 6: return Q == 6 ? 2048 : 3072;
+  default: return 1280;
+  }
+}
+
+// Whether the chain kernel runs a gathered apply of num_cells cells.
+constexpr bool chain_runs(int op, bool f64, int N, int Q, long long num_cells)
+{
+  return chain_pays(op, f64, N, Q) && num_cells >= chain_cells_from(f64, N, Q);
+}
+
 // Cells per workgroup of the fused cell kernel (Q^2 threads per cell):
 // one wave of whole cells up to Q = 8.  At Q = 9 one cell in a 2-wave
 // workgroup would leave 47 of its 128 lanes idle; three cells take 243 of

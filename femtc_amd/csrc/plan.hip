@@ -1,6 +1,6 @@
 // Scatter plans for the continuous operator over a structured cell
-// numbering: the direct scatter of the one-shot apply, an LDS-assembled scatter over 3-D
-// blocks of cells, or the assembled scatter (a cell pass storing every
+// numbering: the direct scatter of the one-shot apply, an LDS-assembled
+// scatter over 3-D blocks of cells, or the assembled scatter (a cell pass storing every
 // cell-dof value without atomics, then a pass summing each global dof;
 // offered when the dofmap is verified to be the structured numbering at
 // plan creation), chosen per (nq, dtype, op) by a default or by timing
@@ -117,14 +117,16 @@ std::vector<Shape> candidates(int nq)
 int key_of(int nq, int dtype, int op) { return (nq * 4 + dtype) * 4 + op; }
 
 // Shape of a plan that has not been autotuned: the direct scatter (the chain
-// kernel where chain_pays), except degree 1 FP64 stiffness and K+M, where
+// kernel where chain_runs), except degree 1 FP64 stiffness and K+M, where
 // blocks of 1 x 2 x 16 cells are the faster of the two.  us per apply of
 // structured meshes, blocked against direct, nq = degree + 1: 155^3 cells at
 // P=1 FP64 stiffness 291 / 313, K+M 333 / 363, mass 164 / 138, FP32 stiffness
 // 241 / 194; 78^3 at P=3 FP64 mass 286 / 199, stiffness 422 / 341, FP32
 // stiffness 324 / 183; 62^3 at P=4 FP64 mass 339 / 210, FP32 K+M 374 / 251.
 // At P = 2..4 every blocked shape that was a default measured 1.2-1.9 times
-// the direct scatter's time.
+// the direct scatter's time, 1.0-2.0 in reader order and 1.5-2.0 with cells
+// shuffled (3e3 to 3e6 dofs); only where the dofs of a structured mesh are in
+// random order, which blocks do not mind, 0.68-0.97.
 Shape default_shape(int degree, int nq, int dtype, int op)
 {
   if (degree == 1 && nq == 2 && dtype == FEMTC_F64 && op != FEMTC_OP_MASS)
@@ -364,7 +366,9 @@ int plan_request(const femtc_plan* pl, int op, int dtype, int nq,
   // shape at nq = degree + 1, 3e6 dofs: lexicographic 1.18-3.4, reader order
   // 1.5-3.5, cells shuffled, along another axis or with rotated local axes
   // 0.97-1.13, plates of one cell 0.98-1.35.
-  const bool direct_eo = s.x == 0 && !chain_pays(op, dtype == FEMTC_F64, r.N, nq);
+  const bool direct_eo =
+      s.x == 0 &&
+      !chain_runs(op, dtype == FEMTC_F64, r.N, nq, pl->num_cells);
   r.eo_tab = (direct_eo || s.x == -1) && nq == r.N ? eo : nullptr;
   r.x = x;
   r.y = y;

@@ -1,6 +1,8 @@
 """The chain kernel behind the one-shot gathered applies: every kind of
 numbering it must merge or must not merge faces for, chains that end short,
-cells straddling waves (Q = 6), overwrite and accumulate, against the oracle.
+cells straddling waves (Q = 6), overwrite and accumulate, against the oracle,
+on boxes of more cells than its count (FROM); the same numberings on a few
+cells, which the atomic kernel runs.
 
 The kernel sums the same products as the atomic scatter in another order, so
 the bars are those of the gathered applies: 1e-12 (FP64), 1e-5 (FP32)."""
@@ -139,56 +141,136 @@ def test_plan_that_was_not_tuned(P, kind):
             assert err <= TOL[dtype], (op, P, kind, dtype, err)
 
 
-def chained_in_part(P, nz, links, seed=3):
-    """(dofmap, number of dofs) of nz cells in a row along z, where cell k
-    (k > 0) shares its left face with cell k-1 only if k is in `links`."""
+# cells from which the chain kernel runs at (P, Q) (FP64 and FP32)
+FROM = {(1, 2): 10240, (1, 3): 24576, (1, 4): 8192, (2, 3): 6144,
+        (2, 4): 6144, (2, 5): 6144, (3, 4): 2048, (3, 5): 5120, (3, 6): 5120,
+        (4, 5): 3072, (4, 6): 4096, (4, 7): 4096, (5, 6): 2048, (5, 7): 3072,
+        (5, 8): 3072, (6, 7): 1280, (6, 8): 1280, (7, 8): 1280}
+CODE = {"mass": F.OP_MASS, "stiffness": F.OP_STIFFNESS, "kpm": F.OP_KPM}
+
+
+def compare(P, Q, dm, ng, ops, accumulate=False):
+    """Gathered applies of every op, both types, per-point and affine geometry,
+    against the oracle."""
     N = P + 1
-    dm = np.empty((nz, N, N, N), dtype=np.int64)
+    C = len(dm) // N ** 3
+    J = O.random_jacobians(5, C)
+    G, Dw = O.geometry_affine(J, Q)
+    tab, x, y0 = O.basis_tables(P, Q), O.uniform(11, ng), O.uniform(12, ng)
+    ddm = torch.from_numpy(dm).cuda()
+    for op in ops:
+        ref = O.global_operator(op, N, Q, tab, x, dm, G, Dw)
+        if accumulate:
+            ref = ref + y0
+        for dtype in (torch.float64, torch.float32):
+            def dev(a):
+                return torch.from_numpy(np.ascontiguousarray(a)).to("cuda",
+                                                                    dtype)
+            cg = torch.empty(C * 7, device="cuda", dtype=dtype)
+            F.geometry_cell(torch.from_numpy(J).cuda(), cg)
+            for affine in (False, True):
+                y = dev(y0)
+                if affine:
+                    F.global_apply_affine(
+                        CODE[op], dev(F.basis_tables_weights(P, Q)), dev(x), y,
+                        ddm, C, P, Q, cg, accumulate=accumulate)
+                else:
+                    F.global_apply(CODE[op], dev(tab), dev(x), y, ddm, C, P, Q,
+                                   G=dev(G), detJw=dev(Dw),
+                                   accumulate=accumulate)
+                torch.cuda.synchronize()
+                got = y.double().cpu().numpy()
+                err = np.linalg.norm(got - ref) / np.linalg.norm(ref)
+                assert err <= TOL[dtype], (op, P, Q, dtype, affine, err)
+
+
+# z-lines shorter than, equal to and longer than a chain, as in SHAPES
+BOXES = [(1, 2, (25, 46, 9)), (2, 3, (31, 40, 5)), (3, 5, (27, 28, 7)),
+         (4, 5, (13, 30, 8)), (5, 6, (19, 22, 5)), (3, 6, (32, 41, 4)),
+         (6, 7, (13, 20, 5)), (7, 8, (18, 18, 4)), (4, 7, (4, 30, 35)),
+         (1, 3, (24, 32, 33))]
+
+
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("P,Q,dims", BOXES)
+def test_numberings_from_the_count(P, Q, dims, kind):
+    assert np.prod(dims) >= FROM[P, Q]
+    compare(P, Q, *numbered(kind, dims, P), ("mass", "stiffness", "kpm"),
+            accumulate=kind in ("reader", "shuffled"))
+
+
+@pytest.mark.parametrize("P,Q", sorted(FROM))
+def test_chain_ends_from_the_count(P, Q):
+    """Last chains of one to three cells, and just short of full."""
+    for more in (1, 3, 31):
+        compare(P, Q, *numbered("lex", (1, 1, FROM[P, Q] + more), P),
+                ("mass",))
+
+
+def operator_kernels(call):
+    """Names of the operator kernels that call() launches."""
+    from torch.profiler import ProfilerActivity, profile
+
+    torch.cuda.synchronize()
+    with profile(activities=[ProfilerActivity.CUDA]) as prof:
+        call()
+        torch.cuda.synchronize()
+    return {e.key for e in prof.key_averages()
+            if "apply_cells<" in e.key or "chain_cells<" in e.key}
+
+
+@pytest.mark.parametrize("P,Q", sorted(FROM))
+def test_kernel_by_count(P, Q):
+    """The atomic kernel below the count, the chain kernel from it on."""
+    N = P + 1
+    for dtype in (torch.float64, torch.float32):
+        at = 0 if (P, Q, dtype) == (1, 4, torch.float32) else FROM[P, Q]
+        for C in (max(at - 1, 1), max(at, 1)):
+            dm = torch.arange(C * N ** 3, device="cuda", dtype=torch.int32)
+            x = torch.ones(C * N ** 3, device="cuda", dtype=dtype)
+            y = torch.empty_like(x)
+            D = torch.ones(C * Q ** 3, device="cuda", dtype=dtype)
+            tab = torch.from_numpy(O.basis_tables(P, Q)).to("cuda", dtype)
+            ran = operator_kernels(lambda: F.global_apply(
+                F.OP_MASS, tab, x, y, dm, C, P, Q, detJw=D))
+            assert len(ran) == 1, ran
+            assert ("chain_cells" in ran.pop()) == (C >= at), (P, Q, C)
+
+
+def chained_in_part(P, nz, rows, links, seed=3):
+    """(dofmap, number of dofs) of `rows` rows of nz cells along z, where cell
+    k (k > 0) of a row shares its left face with cell k-1 only if k is in
+    `links`; dofs in random order."""
+    N = P + 1
+    row = np.empty((nz, N, N, N), dtype=np.int64)
     n = 0
     for k in range(nz):
         first = 0
         if k in links:
-            dm[k, :, :, 0] = dm[k - 1, :, :, P]
+            row[k, :, :, 0] = row[k - 1, :, :, P]
             first = 1
         new = N * N * (N - first)
-        dm[k, :, :, first:] = n + np.arange(new).reshape(N, N, N - first)
+        row[k, :, :, first:] = n + np.arange(new).reshape(N, N, N - first)
         n += new
-    dm = np.random.default_rng(seed).permutation(n)[dm]
-    return np.ascontiguousarray(dm.ravel(), dtype=np.int32), n
+    dm = row[None] + n * np.arange(rows)[:, None, None, None, None]
+    dm = np.random.default_rng(seed).permutation(n * rows)[dm]
+    return np.ascontiguousarray(dm.ravel(), dtype=np.int32), n * rows
 
 
 # the kernel looks at the first two pairs of a chain: merged cells where it
-# takes the whole chain for unmerged, single cells where it merges, and chains
-# of one and two cells (P=5: cells straddling waves)
+# takes the whole chain for unmerged, and single cells where it merges, at every
+# place of a chain (rows of 9 and 34 cells; P=5: cells straddling waves)
 LINKS = [set(), {1}, {2}, {3, 4, 6}, {1, 5}, {2, 4, 6, 8}, {1, 2, 3},
          set(range(1, 40))]
 
 
-@pytest.mark.parametrize("P,Q", [(1, 2), (2, 3), (1, 4), (4, 5), (3, 6),
-                                 (5, 6), (6, 7), (7, 8)])
+@pytest.mark.parametrize("P,Q", [(1, 2), (2, 3), (4, 5), (5, 6), (6, 7),
+                                 (7, 8)])
 @pytest.mark.parametrize("links", LINKS)
 def test_chained_in_part(P, Q, links):
-    N = P + 1
-    for nz in (1, 2, 3, 9, 34):
-        dm, ng = chained_in_part(P, nz, links)
-        J = O.random_jacobians(5, nz)
-        G, Dw = O.geometry_affine(J, Q)
-        tab, x = O.basis_tables(P, Q), O.uniform(11, ng)
-        for op, code, dtype in (("mass", F.OP_MASS, torch.float64),
-                                ("stiffness", F.OP_STIFFNESS, torch.float32)):
-            ref = O.global_operator(op, N, Q, tab, x, dm, G, Dw)
-
-            def dev(a):
-                return torch.from_numpy(np.ascontiguousarray(a)).to("cuda",
-                                                                    dtype)
-            y = torch.empty(ng, device="cuda", dtype=dtype)
-            F.global_apply(code, dev(tab), dev(x), y,
-                           torch.from_numpy(dm).cuda(), nz, P, Q, G=dev(G),
-                           detJw=dev(Dw))
-            torch.cuda.synchronize()
-            got = y.double().cpu().numpy()
-            err = np.linalg.norm(got - ref) / np.linalg.norm(ref)
-            assert err <= TOL[dtype], (op, P, Q, nz, links, err)
+    for nz in (9, 34):
+        rows = -(-FROM[P, Q] // nz)
+        compare(P, Q, *chained_in_part(P, nz, rows, links), ("mass", "kpm"))
 
 
 def test_no_loss_where_nothing_chains():
