@@ -43,7 +43,7 @@
 //   FP32 mass P=3          115 /  42   188 /  55   114 / 114
 //   FP32 stiffness P=4      96 /  54   141 /  55    94 /  90
 //   FP64 mass P=7           66 /  53    89 /  56    70 /  65
-//   affine FP64 K+M P=5     88 /  77   120 /  73    89 / 103
+//   affine FP64 K+M P=5     89 /  71   120 /  71    89 / 103
 //   FP32 mass P=1          299 /  87   298 /  87   622 / 620
 #pragma once
 

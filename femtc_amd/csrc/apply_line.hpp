@@ -969,21 +969,23 @@ int line_launch_op(const ApplyReq& r, int max_lds)
   constexpr int CPB = line_cpb<T, OP, N, Q>();
   const int64_t groups = (r.num_cells + CPB - 1) / CPB;
   const int64_t grid = std::min<int64_t>(groups, 16384);
-  if constexpr (line_staged<T, OP, N, Q>())
+  if constexpr (!line_staged<T, OP, N, Q>())
+    return line_launch_form<T, OP, N, Q, false>(r, grid);
+  else if constexpr (line_staged_from<T, OP, N, Q>() == 0)
+    return line_launch_form<T, OP, N, Q, true>(r, grid);
+  else
   {
-    constexpr int FROM = line_staged_from<T, OP, N, Q>();
-    if constexpr (FROM == 0)
-      return line_launch_form<T, OP, N, Q, true>(r, grid);
     int dev = 0, cus = 0;
     if (hipGetDevice(&dev) == hipSuccess &&
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount,
                               dev) == hipSuccess &&
-        cus > 0 && 4 * groups >= (int64_t)FROM * cus)
+        cus > 0 &&
+        4 * groups >= (int64_t)line_staged_from<T, OP, N, Q>() * cus)
       // one workgroup of two staged cells is resident on a CU (10 waves or
       // more, over 96 VGPRs) and takes all of the CU's pairs
       return line_launch_form<T, OP, N, Q, true>(r, CPB == 2 ? cus : grid);
+    return line_launch_form<T, OP, N, Q, false>(r, grid);
   }
-  return line_launch_form<T, OP, N, Q, false>(r, grid);
 }
 
 template <typename T, int OP, int N, int Q>

@@ -1203,8 +1203,8 @@ int sync_write(femtc_solver* S, void* dev, const void* host, size_t bytes)
   } while (0)
 
 // check_every CG iterations in precision V, queued on stream s: operator
-// (with the p.Ap energies), update (with alpha), p-update (with beta).  Every kernel
-// returns at once after the state's `done` is set.
+// (with the p.Ap energies), update (with alpha), p-update (with beta).  Every
+// kernel returns at once after the state's `done` is set.
 template <typename V>
 int enqueue_batch(femtc_solver* S, hipStream_t s)
 {

@@ -22,8 +22,8 @@ TOL = {torch.float64: 1e-12, torch.float32: 1e-5}
 
 
 def _pairs_apart():
-    # four pairs of cells per CU: from there on a workgroup of two staged
-    # cells takes several pairs
+    # four pairs of cells per CU: workgroups of two staged cells (from three
+    # pairs per CU on) take several pairs
     return 8 * torch.cuda.get_device_properties(0).multi_processor_count
 
 
